@@ -75,6 +75,15 @@ int hip_qmm_quantize_q8_1_planar(const float *x, int64_t K, int64_t ncols, int64
  * MMQ spreads K over several workgroups. */
 size_t hip_qmm_mul_mat_workspace_size(int type, int64_t K, int64_t nrows, int64_t ncols);
 
+/* Bytes of workspace with which hip_qmm_mul_mat runs its fastest kernel for this
+ * shape: at least hip_qmm_mul_mat_workspace_size, more where the f16 GEMM
+ * (mmq_f16.hip, large grids of Q4_K, Q5_K and Q6_K above 32 columns) takes the
+ * columns as panels.  With less, down to hip_qmm_mul_mat_workspace_size, the
+ * int8 MMQ runs.  hip_qmm_mul_mat_glu_workspace_preferred: the same for
+ * hip_qmm_mul_mat_glu. */
+size_t hip_qmm_mul_mat_workspace_preferred(int type, int64_t K, int64_t nrows, int64_t ncols);
+size_t hip_qmm_mul_mat_glu_workspace_preferred(int type, int64_t K, int64_t nrows, int64_t ncols);
+
 /* 1 if hip_qmm_mul_mat runs an MMQ kernel (the few-column GEMM or the tile)
  * rather than the GEMV for this shape on 16-byte-aligned rows, else 0 (the
  * shape rules that hip_qmm_mul_mat_workspace_size applies).  No counterpart

@@ -21,6 +21,22 @@ bool few_cols_type(int type, int64_t K, int64_t nrows, int64_t ncols);
 // mmq_few.hip: whether it takes these weight rows
 bool mmq_few_takes(int type, int64_t K, const void *w, int64_t row_stride);
 
+// mmq.hip: its weight checks, and the sum of K-split partials
+int mmq_check_weights(int type, const void *w, int64_t K, int64_t row_stride);
+int mmq_add_partials(const float *partial, int split, int64_t nrows, int64_t ncols, float *dst, int64_t dst_col_stride,
+                     hipStream_t s);
+// mmq_f16.hip: the large-grid Q4_K / Q5_K / Q6_K GEMM on f16 matrix cores
+struct MmqF16Plan {
+    bool use, wide;
+    int split;
+};
+MmqF16Plan mmq_f16_plan(int type, int64_t K, int64_t nrows, int64_t ncols, bool glu);
+size_t mmq_f16_panel_bytes(int64_t K, int64_t ncols);
+int mmq_f16_quantize(const float *x, int64_t K, int64_t ncols, int64_t x_col_stride, void *panels, hipStream_t s);
+int mmq_f16_launch(int type, bool wide, const void *w, int64_t K, int64_t nrows, int64_t row_stride,
+                   const void *panels, int64_t ncols, float *dst, int64_t dst_col_stride, float *partial, int split,
+                   const MmqGlu &glu, hipStream_t s);
+
 // gemv.hip: 2-4 f32 columns (or twice the kernel's columns as two grid rows)
 // through the quantize-in-GEMV kernel, or hipErrorNotSupported for shapes it
 // does not take.
@@ -128,6 +144,34 @@ size_t glu_unfused_bytes(int type, int64_t K, int64_t nrows, int64_t ncols) {
     return align256((size_t)2 * (size_t)nrows * (size_t)ncols * sizeof(float)) +
            hip_qmm_mul_mat_workspace_size(type, K, nrows, ncols);
 }
+// Workspace of the f16 route: the panels, then the K-split partials.
+size_t f16_bytes(const MmqF16Plan &pl, int64_t K, int64_t nrows, int64_t ncols) {
+    const size_t partials = pl.split > 1 ? (size_t)pl.split * (size_t)nrows * (size_t)ncols * sizeof(float) : 0;
+    return align256(mmq_f16_panel_bytes(K, ncols)) + partials;
+}
+
+// The f16 route of a product (w_gate null) or of gate/up/GLU, or
+// hipErrorNotSupported where it does not apply: a shape that the plan leaves to
+// the int8 kernels, operands they would check further, or a workspace that does
+// not hold the panels (they are twice the Q8_1 planes, so a caller's workspace of
+// the required size keeps the int8 kernels).
+int f16_route(int type, const void *w, const void *w_gate, int64_t K, int64_t nrows, int64_t row_stride,
+              const float *x, int64_t ncols, int64_t x_col_stride, int glu_op, float glu_alpha, float glu_limit,
+              float *dst, int64_t dst_col_stride, void *workspace, size_t workspace_size, void *stream) {
+    const MmqF16Plan pl = mmq_f16_plan(type, K, nrows, ncols, w_gate != nullptr);
+    if (!pl.use || !w || (uintptr_t)x % 16 || x_col_stride % 4 || dst_col_stride < nrows ||
+        mmq_check_weights(type, w, K, row_stride) || (w_gate && mmq_check_weights(type, w_gate, K, row_stride)) ||
+        workspace_size < f16_bytes(pl, K, nrows, ncols))
+        return (int)hipErrorNotSupported;
+    hipStream_t s = (hipStream_t)stream;
+    float *partial = pl.split > 1 ? (float *)((uint8_t *)workspace + align256(mmq_f16_panel_bytes(K, ncols))) : nullptr;
+    const MmqGlu glu{(const uint8_t *)w_gate, glu_op, glu_alpha, glu_limit};
+    if (int e = mmq_f16_quantize(x, K, ncols, x_col_stride, workspace, s)) return e;
+    if (int e = mmq_f16_launch(type, pl.wide, w, K, nrows, row_stride, workspace, ncols, dst, dst_col_stride, partial,
+                               pl.split, glu, s))
+        return e;
+    return partial ? mmq_add_partials(partial, pl.split, nrows, ncols, dst, dst_col_stride, s) : 0;
+}
 }  // namespace
 
 extern "C" int hip_qmm_version(void) { return (0 << 16) | 1; }
@@ -139,6 +183,13 @@ extern "C" size_t hip_qmm_mul_mat_workspace_size(int type, int64_t K, int64_t nr
     size_t n = q8_1_bytes(K, ncols);
     if (nrows > 0 && use_mmq(type, K, nrows, ncols)) n = align256(n) + hip_qmm_mmq_workspace_size(type, K, nrows, ncols);
     return n;
+}
+
+extern "C" size_t hip_qmm_mul_mat_workspace_preferred(int type, int64_t K, int64_t nrows, int64_t ncols) {
+    const size_t need = hip_qmm_mul_mat_workspace_size(type, K, nrows, ncols);
+    const MmqF16Plan pl = mmq_f16_plan(type, K, nrows, ncols, false);
+    const size_t f16 = pl.use ? f16_bytes(pl, K, nrows, ncols) : 0;
+    return f16 > need ? f16 : need;
 }
 
 extern "C" int hip_qmm_mul_mat_uses_mmq(int type, int64_t K, int64_t nrows, int64_t ncols) {
@@ -167,6 +218,11 @@ extern "C" int hip_qmm_mul_mat(int type, const void *w, int64_t K, int64_t nrows
     if (ncols >= 2 && ncols <= 8 && !use_mmq_rows(type, K, nrows, ncols, w, row_stride)) {
         const int e = qmm_mul_mat_fx_cols(type, w, K, nrows, row_stride, x, ncols, x_col_stride, dst, dst_col_stride,
                                           stream);
+        if (e != (int)hipErrorNotSupported) return e;
+    }
+    if (ncols > 8) {
+        const int e = f16_route(type, w, nullptr, K, nrows, row_stride, x, ncols, x_col_stride, 0, 0.0f, 0.0f, dst,
+                                dst_col_stride, workspace, workspace_size, stream);
         if (e != (int)hipErrorNotSupported) return e;
     }
     const int64_t Kp = pad_k(K);
@@ -202,6 +258,14 @@ extern "C" size_t hip_qmm_mul_mat_glu_workspace_size(int type, int64_t K, int64_
     return glu_unfused_bytes(type, K, nrows, ncols);  // one column: only used when the fused GEMV cannot run
 }
 
+extern "C" size_t hip_qmm_mul_mat_glu_workspace_preferred(int type, int64_t K, int64_t nrows, int64_t ncols) {
+    const size_t need = hip_qmm_mul_mat_glu_workspace_size(type, K, nrows, ncols);
+    if (K <= 0 || nrows <= 0 || ncols <= 0 || !glu_fuses_mmq(type, K, nrows, ncols)) return need;
+    const MmqF16Plan pl = mmq_f16_plan(type, K, nrows, ncols, true);
+    const size_t f16 = pl.use ? f16_bytes(pl, K, nrows, ncols) : 0;
+    return f16 > need ? f16 : need;
+}
+
 extern "C" int hip_qmm_mul_mat_glu(int type, const void *w, const void *w_gate, int64_t K, int64_t nrows,
                                    int64_t row_stride, const float *x, int64_t ncols, int64_t x_col_stride,
                                    int glu_op, float glu_alpha, float glu_limit, float *dst, int64_t dst_col_stride,
@@ -216,6 +280,9 @@ extern "C" int hip_qmm_mul_mat_glu(int type, const void *w, const void *w_gate, 
         workspace_size < hip_qmm_mul_mat_glu_workspace_size(type, K, nrows, ncols))
         return (int)hipErrorInvalidValue;
     if (glu_fuses_mmq(type, K, nrows, ncols)) {
+        const int f16 = f16_route(type, w, w_gate, K, nrows, row_stride, x, ncols, x_col_stride, glu_op, glu_alpha,
+                                  glu_limit, dst, dst_col_stride, workspace, workspace_size, stream);
+        if (f16 != (int)hipErrorNotSupported) return f16;
         const int64_t Kp = pad_k(K);
         int8_t *qs = (int8_t *)workspace;
         void *ds = (uint8_t *)workspace + ncols * Kp;

@@ -518,7 +518,7 @@ bool run_mul_mat(BackendCtx *ctx, const ggml_tensor *node) {
     }
     // One batch, or more than 8 columns: the op per (i2, i3) slice (its
     // MMQ takes one weight matrix per launch).
-    const size_t need = hip_qmm_mul_mat_workspace_size(a->type, K, M, N);
+    const size_t need = hip_qmm_mul_mat_workspace_preferred(a->type, K, M, N);
     void *ws = workspace(ctx, need);
     for (int64_t i3 = 0; i3 < b->ne[3]; ++i3)
         for (int64_t i2 = 0; i2 < b->ne[2]; ++i2) {
@@ -859,7 +859,7 @@ bool launch_fused_mmq(BackendCtx *ctx, const ggml_tensor *up, const ggml_tensor 
     const int64_t K = w->ne[0], M = w->ne[1], N = x->ne[1];
     if (overlaps(out->data, nbytes(out), x->data, nbytes(x)) || lands_on_weights(out->data, nbytes(out), up, gate))
         return false;
-    void *ws = workspace(ctx, hip_qmm_mul_mat_glu_workspace_size(w->type, K, M, N));
+    void *ws = workspace(ctx, hip_qmm_mul_mat_glu_workspace_preferred(w->type, K, M, N));
     const int rc = hip_qmm_mul_mat_glu(w->type, w->data, gate->src[0]->data, K, M, (int64_t)w->nb[1],
                                        static_cast<const float *>(x->data), N, (int64_t)(x->nb[1] / 4),
                                        out->op_params[0], op_param_f32(out, 2), op_param_f32(out, 3),

@@ -904,6 +904,15 @@ bool few_cols_type(int type, int64_t K, int64_t nrows, int64_t ncols) {
     return true;
 }
 
+// For api.hip's f16 route: the weight checks of this dispatch, and the sum of K-split partials.
+int mmq_check_weights(int type, const void *w, int64_t K, int64_t row_stride) {
+    return check_weights(type, w, K, row_stride);
+}
+int mmq_add_partials(const float *partial, int split, int64_t nrows, int64_t ncols, float *dst, int64_t dst_col_stride,
+                     hipStream_t s) {
+    return launch_reduce(partial, split, nrows, ncols, dst, dst_col_stride, s);
+}
+
 extern "C" int hip_qmm_mmq_split_k(int type, int64_t K, int64_t nrows, int64_t ncols) {
     if (K <= 0 || nrows <= 0 || ncols <= 0) return 1;
     return few_cols_type(type, K, nrows, ncols) ? mmq_few_split_k(K, nrows) : split_std(type, K, nrows, ncols);

@@ -45,6 +45,9 @@ def lib():
         L.hip_qmm_quantize_q8_1_planar.argtypes = [vp, i64, i64, i64, vp, vp, vp]
         L.hip_qmm_mul_mat_workspace_size.restype = ctypes.c_size_t
         L.hip_qmm_mul_mat_workspace_size.argtypes = [i32, i64, i64, i64]
+        for name in ("hip_qmm_mul_mat_workspace_preferred", "hip_qmm_mul_mat_glu_workspace_preferred"):
+            getattr(L, name).restype = ctypes.c_size_t
+            getattr(L, name).argtypes = [i32, i64, i64, i64]
         L.hip_qmm_mul_mat_uses_mmq.argtypes = [i32, i64, i64, i64]
         L.hip_qmm_mul_mat_per_column.argtypes = [i32, i64, i64, i64]
         L.hip_qmm_mul_mat_vec.restype = i32
@@ -398,11 +401,13 @@ def mul_mat_glu(qtype, w: torch.Tensor, w_gate: torch.Tensor, x: torch.Tensor, g
     n, K = x.shape
     t, nrows, rs = _glu_weights(qtype, w, w_gate, K)
     op = GLU_OPS[glu] if isinstance(glu, str) else int(glu)
-    need = int(lib().hip_qmm_mul_mat_glu_workspace_size(t, K, nrows, n))
     if workspace is None:
-        workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
-    elif workspace.numel() < need:
-        raise HipQmmError(f"workspace too small: {workspace.numel()} < {need}")
+        size = int(lib().hip_qmm_mul_mat_glu_workspace_preferred(t, K, nrows, n))
+        workspace = torch.empty(max(size, 1), dtype=torch.uint8, device=x.device)
+    else:
+        need = int(lib().hip_qmm_mul_mat_glu_workspace_size(t, K, nrows, n))
+        if workspace.numel() < need:
+            raise HipQmmError(f"workspace too small: {workspace.numel()} < {need}")
     out = torch.empty((n, nrows), dtype=torch.float32, device=x.device) if out is None else out
     _check(lib().hip_qmm_mul_mat_glu(t, _ptr(w), _ptr(w_gate), K, nrows, rs, _ptr(x), n, x.stride(0), op, alpha,
                                      limit, _ptr(out), out.stride(0), _ptr(workspace), workspace.numel(), _stream()),
@@ -456,11 +461,13 @@ def mul_mat(qtype, w: torch.Tensor, x: torch.Tensor, out=None, workspace=None):
         raise HipQmmError("x must be a 2-D float32 tensor [ncols, K]")
     n, K = x.shape
     t, nrows, rs = _weight_args(qtype, w, K)
-    need = workspace_size(t, K, n, nrows)
     if workspace is None:
-        workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
-    elif workspace.numel() < need:
-        raise HipQmmError(f"workspace too small: {workspace.numel()} < {need}")
+        size = int(lib().hip_qmm_mul_mat_workspace_preferred(t, K, nrows, n))
+        workspace = torch.empty(size, dtype=torch.uint8, device=x.device)
+    else:
+        need = workspace_size(t, K, n, nrows)
+        if workspace.numel() < need:
+            raise HipQmmError(f"workspace too small: {workspace.numel()} < {need}")
     out = torch.empty((n, nrows), dtype=torch.float32, device=x.device) if out is None else out
     _check(lib().hip_qmm_mul_mat(t, _ptr(w), K, nrows, rs, _ptr(x), n, x.stride(0), _ptr(out), out.stride(0),
                                  _ptr(workspace), workspace.numel(), _stream()), "hip_qmm_mul_mat")
