@@ -391,8 +391,9 @@ int hip_qmm_mmq_grouped_glu(int type, const void *w, const void *w_gate, int64_t
 /* Bytes of workspace hip_qmm_mul_mat_glu needs (none for one column when the fused GEMV takes it). */
 size_t hip_qmm_mul_mat_glu_workspace_size(int type, int64_t K, int64_t nrows, int64_t ncols);
 
-/* 1 if hip_qmm_mul_mat_glu runs the fused MMQ for this shape (the products
- * would each run the MMQ tile kernel), else 0: the reference's
+/* 1 if hip_qmm_mul_mat_glu runs a fused MMQ for this shape (the products
+ * would each run the MMQ tile kernel, or, above 8 columns, the few-column GEMM
+ * takes both weights in one launch), else 0: the reference's
  * shouldFuseMulMatQ (src/ggml/cuda/mulmat.zig:548-571) for this backend. */
 int hip_qmm_mul_mat_glu_fused(int type, int64_t K, int64_t nrows, int64_t ncols);
 
@@ -402,10 +403,14 @@ int hip_qmm_mul_mat_glu_fused(int type, int64_t K, int64_t nrows, int64_t ncols)
  * src/ggml/cuda/mulmat.zig:548-571): dst[c][r] = glu(glu_op, (Wg . x_c)[r], (W . x_c)[r])
  * for ncols f32 columns x[c*x_col_stride + k].  One column:
  * hip_qmm_mul_mat_vec_fused.  Where the unfused products would run the MMQ
- * tile kernel: one Q8_1 quantization and hip_qmm_mmq_glu.  Between (the
- * GEMV's and the few-column kernel's column counts, which the reference does
- * not fuse either): the two hip_qmm_mul_mat products into the workspace and
- * hip_qmm_glu_f32, as the unfused graph runs.  Limits of hip_qmm_mul_mat.
+ * tile kernel: one Q8_1 quantization and hip_qmm_mmq_glu (or the f16 GEMM, see
+ * hip_qmm_mul_mat_glu_workspace_preferred).  Between (the GEMV's and the
+ * few-column kernel's column counts): on 4096 rows and more, one quantization
+ * and the few-column GEMM on both weights with the GLU in its epilogue, whose
+ * sums differ from the separate products' in fp32 rounding only; on smaller
+ * matrices and a few measured exceptions, the two hip_qmm_mul_mat products into
+ * the workspace and hip_qmm_glu_f32, as the unfused graph runs.  Limits of
+ * hip_qmm_mul_mat.
  */
 int hip_qmm_mul_mat_glu(int type, const void *w, const void *w_gate, int64_t K, int64_t nrows, int64_t row_stride,
                         const float *x, int64_t ncols, int64_t x_col_stride, int glu_op, float glu_alpha,

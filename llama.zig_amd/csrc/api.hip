@@ -21,6 +21,9 @@ bool few_cols_type(int type, int64_t K, int64_t nrows, int64_t ncols);
 // mmq_few.hip: whether it takes these weight rows
 bool mmq_few_takes(int type, int64_t K, const void *w, int64_t row_stride);
 
+int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *yqs,
+                   const void *yds, int64_t ncols, float *dst, int64_t dst_col_stride, int split, float *partial,
+                   const MmqGlu &glu, hipStream_t s);
 // mmq.hip: its weight checks, and the sum of K-split partials
 int mmq_check_weights(int type, const void *w, int64_t K, int64_t row_stride);
 int mmq_add_partials(const float *partial, int split, int64_t nrows, int64_t ncols, float *dst, int64_t dst_col_stride,
@@ -138,6 +141,34 @@ bool glu_fuses_mmq(int type, int64_t K, int64_t nrows, int64_t ncols) {
     return ncols >= 2 && use_mmq(type, K, nrows, ncols) && !few_cols_type(type, K, nrows, ncols);
 }
 
+// Whether gate/up/GLU over ncols columns runs the few-column kernel on both
+// weights with the GLU in its epilogue (one quantizer and one launch) rather
+// than two products and the GLU kernel (two quantizers, two GEMVs or few-column
+// GEMMs with their K-split reductions, one GLU).  Both weights' rows give the
+// grid twice the workgroups, so it needs no K split from 4096 rows on.  Measured
+// (whole call, us, graph-timed, unfused -> fused): Q4_K 14336x4096 at 2 / 4 / 9 /
+// 16 / 32 columns 25.1 -> 21.3, 27.9 -> 20.8, 31.3 -> 22.1, 32.6 -> 22.6, 43.2 ->
+// 30.1; 8192x4096 at 4 / 16 25.7 -> 13.9, 28.7 -> 14.5; 4096x4096 at 4 / 8 16.1 ->
+// 12.7, 21.2 -> 12.7; Q5_K 14336x4096 at 13 34.6 -> 25.6; Q6_K at 4 44.1 -> 33.3;
+// Q8_0 at 4 39.1 -> 30.1; Q4_0 at 8 34.8 -> 25.2; IQ4_XS at 8 38.4 -> 27.6.  The
+// unfused route stays where it measured level or faster: few columns of small or
+// long-row matrices, whose one-launch GEMVs have no quantizer (Q4_K 4096x4096 at
+// 2 11.7 against 13.0; Q6_K 5120x8192 at 2 32.5 / 34.0; Q4_0 4096x8192 at 4 22.0 /
+// 24.6; IQ4_XS 14336x14336 at 2 70.2 / 78.5, 5120x8192 at 3 26.3 / 26.6), and
+// below 4096 rows or 12M weights, where the unsplit grid is too small (Q4_K
+// 1024x8192 at 4 16.4 against 19.6).
+bool glu_few(int type, int64_t K, int64_t nrows, int64_t ncols) {
+    if (K % 256 != 0 || nrows < 4096 || nrows * K < ((int64_t)12 << 20) || !few_cols_type(type, K, nrows, ncols))
+        return false;
+    if (nrows < 5120) return ncols >= (type == TYPE_Q4_0 || type == TYPE_IQ4_XS ? 8 : 4);
+    switch (type) {
+    case TYPE_Q6_K:
+    case TYPE_Q4_0: return ncols >= 3;
+    case TYPE_IQ4_XS: return ncols >= 4;
+    default: return ncols >= 2;
+    }
+}
+
 // The unfused gate/up/GLU's workspace: the gate and up products, then
 // hip_qmm_mul_mat's own workspace.
 size_t glu_unfused_bytes(int type, int64_t K, int64_t nrows, int64_t ncols) {
@@ -249,7 +280,9 @@ extern "C" int hip_qmm_mul_mat(int type, const void *w, int64_t K, int64_t nrows
 }
 
 extern "C" int hip_qmm_mul_mat_glu_fused(int type, int64_t K, int64_t nrows, int64_t ncols) {
-    return K > 0 && nrows > 0 && glu_fuses_mmq(type, K, nrows, ncols) ? 1 : 0;
+    return K > 0 && nrows > 0 && (glu_fuses_mmq(type, K, nrows, ncols) || (ncols > 8 && glu_few(type, K, nrows, ncols)))
+               ? 1
+               : 0;
 }
 
 extern "C" size_t hip_qmm_mul_mat_glu_workspace_size(int type, int64_t K, int64_t nrows, int64_t ncols) {
@@ -289,6 +322,17 @@ extern "C" int hip_qmm_mul_mat_glu(int type, const void *w, const void *w_gate, 
         if (int e = hip_qmm_quantize_q8_1_planar(x, K, ncols, x_col_stride, qs, ds, stream)) return e;
         return hip_qmm_mmq_glu(type, w, w_gate, K, nrows, row_stride, qs, ds, ncols, glu_op, glu_alpha, glu_limit,
                                dst, dst_col_stride, stream);
+    }
+    if (glu_few(type, K, nrows, ncols) && mmq_few_takes(type, K, w, row_stride) &&
+        mmq_few_takes(type, K, w_gate, row_stride) && !mmq_check_weights(type, w, K, row_stride) &&
+        !mmq_check_weights(type, w_gate, K, row_stride) && dst_col_stride >= nrows) {
+        const int64_t Kp = pad_k(K);
+        int8_t *qs = (int8_t *)workspace;
+        void *ds = (uint8_t *)workspace + ncols * Kp;
+        if (int e = hip_qmm_quantize_q8_1_planar(x, K, ncols, x_col_stride, qs, ds, stream)) return e;
+        const MmqGlu glu{(const uint8_t *)w_gate, glu_op, glu_alpha, glu_limit};
+        return mmq_few_launch(type, w, K, nrows, row_stride, qs, ds, ncols, dst, dst_col_stride, 1, nullptr, glu,
+                              (hipStream_t)stream);
     }
     float *g = (float *)workspace, *u = g + nrows * ncols;
     const size_t off = align256((size_t)2 * (size_t)nrows * (size_t)ncols * sizeof(float));

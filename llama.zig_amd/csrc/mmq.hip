@@ -62,7 +62,7 @@ int mmq_few_split_k(int64_t K, int64_t nrows);
 bool mmq_few_takes(int type, int64_t K, const void *w, int64_t row_stride);
 int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *yqs,
                    const void *yds, int64_t ncols, float *dst, int64_t dst_col_stride, int split, float *partial,
-                   hipStream_t s);
+                   const MmqGlu &glu, hipStream_t s);
 
 namespace {
 
@@ -945,7 +945,7 @@ extern "C" int hip_qmm_mmq(int type, const void *w, int64_t K, int64_t nrows, in
     hipStream_t s = (hipStream_t)stream;
     if (few) {
         if (int e = mmq_few_launch(type, w, K, nrows, row_stride, y_qs, y_ds, ncols, dst, dst_col_stride, split,
-                                   partial, s))
+                                   partial, MmqGlu{}, s))
             return e;
         return split > 1 ? launch_reduce(partial, split, nrows, ncols, dst, dst_col_stride, s) : 0;
     }

@@ -53,6 +53,14 @@
 // Operand reads at 2-byte alignment in LDS take two byte funnel shifts of
 // three aligned dwords.
 //
+// Gate/up/GLU (MmqGlu): a 64-row tile holds 32 output rows, tile row t reading the
+// gate (t % 4 < 2) or up weights of output row mmq_glu_tile_row(t), so a lane's
+// four rows of a column are gate and up of two output rows and the epilogue
+// writes the GLU without an exchange.  Unsplit: both weights' rows fill the grid.
+// Two rings of one K half each share a CU only up to 256 workgroups; the 448 of
+// 2 x 14336 rows run one ring each, three to a CU, and read 66 MB in 18.5 us at
+// 4-16 columns where two plain launches take 2 x 11.8 us and the GLU pass 3.5.
+//
 // 16x16 MFMA operand convention: lane l supplies row (l % 16) of A and column
 // (l % 16) of B over the K-slice [(l / 16) * K/4, +K/4); the result value i of
 // lane l is row 4*(l/16) + i, column l % 16.
@@ -214,11 +222,11 @@ constexpr int few_occupancy(int nst, int kh = 1) { return 163840 / (kh * nst * F
 // step count a multiple of KH), so two waves with independent work share a
 // SIMD; the groups meet at every ring barrier (equal step counts) and add
 // their sums through LDS at the end, group 0 first (deterministic).
-template <int TYPE, int NST, int NW, int NCT, bool PACK, int KH>
+template <int TYPE, int NST, int NW, int NCT, bool PACK, int KH, bool FUSED>
 __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TYPE, NW, NCT>(NST, KH))) void mmq_few_kernel(
     const uint8_t *__restrict__ w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *__restrict__ yqs,
     const uint32_t *__restrict__ yds, int ncols, float *__restrict__ dst, int64_t dst_col_stride,
-    float *__restrict__ partial) {
+    float *__restrict__ partial, MmqGlu glu) {
     static_assert(!PACK || (NCT == 1 && (TYPE == TYPE_Q4_K || TYPE == TYPE_Q5_K || TYPE == TYPE_Q6_K)),
                   "packed: one tile, K-quants");
     using G = FewGeo<TYPE, NW, NCT>;
@@ -238,7 +246,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
     const int kh = wave_all / NW, wave = wave_all - kh * NW;  // K half, wave within it
     uint8_t(*st)[G::STAGE] = rings[kh];
     const int li = lane & 15, kq = lane >> 4;
-    const int64_t row0 = (int64_t)blockIdx.x * G::BM;
+    const int64_t row0 = (int64_t)blockIdx.x * G::BM;  // FUSED: of the gate and up rows together
     const int nkb = (int)(K / QK_K);
     const int gz = (int)gridDim.z, z = (int)blockIdx.z;
     const int kz0 = (int)((int64_t)nkb * z / gz), kz1 = (int)((int64_t)nkb * (z + 1) / gz);
@@ -255,8 +263,9 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
         const int pos = (q < FNQ ? q : 0) * 1024 + lane * 16;
         if (pos < FA) {
             const int r = pos / WROW, off = pos - r * WROW;
-            const int64_t grow = row0 + r < nrows ? row0 + r : nrows - 1;  // rows past the end: duplicates
-            src[i] = w + grow * row_stride + off;
+            const int64_t trow = FUSED ? row0 / 2 + mmq_glu_tile_row(r) : row0 + r;
+            const int64_t grow = trow < nrows ? trow : nrows - 1;  // rows past the end: duplicates
+            src[i] = (FUSED && (r & 2) == 0 ? glu.gate : w) + grow * row_stride + off;
             kstep[i] = 0;  // the weights' step offset is FF::aoff
         } else if (pos < FA + FB) {
             const int p = pos - FA, n = p >> 8, c = ((p >> 4) & 15) ^ (n & 15);
@@ -281,9 +290,27 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
         }
     };
 
-    v4f acc[NCT];
+    // The sums over K-steps.  A fused launch runs unsplit, so a lane adds up to 56
+    // steps in a row, which would round further from the f64 value than the 64-lane
+    // tree of the GEMV it replaces (4.4e-7 against 2.7e-7 of the result at K =
+    // 4096): it keeps the rounding errors of these additions (Knuth's two-sum) and
+    // adds them at the end (2.4e-7).  m is the min term's -dmin and P its sum.
+    v4f acc[NCT], lost[NCT];
 #pragma unroll
-    for (int j = 0; j < NCT; ++j) acc[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < NCT; ++j) acc[j] = lost[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    auto add_sum = [&](int j, int v, float t) {
+        const float a = acc[j][v], s = a + t, b = s - a;
+        lost[j][v] += (a - (s - b)) + (t - b);
+        acc[j][v] = s;
+    };
+    auto add_step = [&](int j, int v, float d, float sum) {
+        if constexpr (FUSED) add_sum(j, v, d * sum);
+        else acc[j][v] = fmaf(d, sum, acc[j][v]);
+    };
+    auto add_step_min = [&](int j, int v, float d, float sum, float m, float P) {
+        if constexpr (FUSED) add_sum(j, v, fmaf(d, sum, m * P));
+        else acc[j][v] = fmaf(d, sum, fmaf(m, P, acc[j][v]));
+    };
     // K-slot carriers: slot 0 and 2 of the scale MFMA live in lanes 0-15,
     // slots 0-7 of the min MFMA in lanes 0-31; the other lanes' A values are
     // zero, so their (finite) B values add nothing.
@@ -315,6 +342,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
         uint4 dh0[NCT], dh1[NCT];
 #pragma unroll
         for (int j = 0; j < NCT; ++j) col_headers(st, j, bcol[j], dh0[j], dh1[j]);
+        v4f accb[NCT];
 #pragma unroll
         for (int g = 0; g < 8; ++g) {
             // Q8_0: the lane's 8 codes of block g; Q4_0: byte j of the 16 holds
@@ -339,8 +367,17 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
                 const v4f zf = {0.0f, 0.0f, 0.0f, 0.0f};
                 const v4f SC = __builtin_amdgcn_mfma_f32_16x16x16f16(sa, scale_b(g, dh0[j], dh1[j]), zf, 0, 0, 0);
 #pragma unroll
-                for (int v = 0; v < 4; ++v) acc[j][v] = fmaf((float)S[v], SC[v], acc[j][v]);
+                for (int v = 0; v < 4; ++v) {
+                    if constexpr (FUSED) accb[j][v] = g == 0 ? (float)S[v] * SC[v] : fmaf((float)S[v], SC[v], accb[j][v]);
+                    else acc[j][v] = fmaf((float)S[v], SC[v], acc[j][v]);
+                }
             }
+        }
+        if constexpr (FUSED) {
+#pragma unroll
+            for (int j = 0; j < NCT; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) add_sum(j, v, accb[j][v]);
         }
     };
 
@@ -392,7 +429,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
             const uint8_t *ob = st + (wave * 16 + 4 * kq + v) * WROW + delta;
             const float d = h2f((uint32_t)*reinterpret_cast<const uint16_t *>(ob + 208));
 #pragma unroll
-            for (int j = 0; j < NCT; ++j) acc[j][v] = fmaf(d, accb[j][v], acc[j][v]);
+            for (int j = 0; j < NCT; ++j) add_step(j, v, d, accb[j][v]);
         }
     };
 
@@ -438,7 +475,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
             const uint8_t *ob = st + (wave * 16 + 4 * kq + v) * WROW + delta;
             const float d = h2f((uint32_t)*reinterpret_cast<const uint16_t *>(ob));
 #pragma unroll
-            for (int j = 0; j < NCT; ++j) acc[j][v] = fmaf(d, accb[j][v], acc[j][v]);
+            for (int j = 0; j < NCT; ++j) add_step(j, v, d, accb[j][v]);
         }
     };
 
@@ -514,7 +551,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
             const v4f zf = {0.0f, 0.0f, 0.0f, 0.0f};
             const v4f P = __builtin_amdgcn_mfma_f32_16x16x16f16(am, bm, zf, 0, 0, 0);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) acc[j][v] = fmaf(dr[v], accb[j][v], fmaf(dn[v], P[v], acc[j][v]));
+            for (int v = 0; v < 4; ++v) add_step_min(j, v, dr[v], accb[j][v], dn[v], P[v]);
         }
     };
 
@@ -594,7 +631,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const uint32_t dd = *reinterpret_cast<const uint32_t *>(st + (wave * 16 + 4 * kq + v) * WROW);
-            acc[0][v] = fmaf(h2f(dd), accb[v], fmaf(-h2f(dd >> 16), P[v], acc[0][v]));
+            add_step_min(0, v, h2f(dd), accb[v], -h2f(dd >> 16), P[v]);
         }
     };
 
@@ -646,7 +683,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
         for (int v = 0; v < 4; ++v) {
             const uint8_t *ob = st + (wave * 16 + 4 * kq + v) * WROW + delta;
             const float d = h2f((uint32_t)*reinterpret_cast<const uint16_t *>(ob + 208));
-            acc[0][v] = fmaf(d, accb[v], acc[0][v]);
+            add_step(0, v, d, accb[v]);
         }
     };
 
@@ -672,6 +709,10 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
             if (++kb >= kb1) break;
         }
     }
+    if constexpr (FUSED) {
+#pragma unroll
+        for (int j = 0; j < NCT; ++j) acc[j] += lost[j];
+    }
     if constexpr (KH > 1) {
         // every wave's ring reads (and transfers: the last wait was vmcnt(0))
         // are done; K half 1 hands its sums to half 0 through the first stage
@@ -687,29 +728,32 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
         for (int j = 0; j < NCT; ++j) acc[j] += part[(j * NW + wave) * 64 + lane];
     }
 
+    // a lane's four rows of a column; fused, gate (v = 0, 1) and up (v = 2, 3) of two output rows
+    auto store_rows = [&](float *o, const v4f &a) {
+        const int64_t r0 = row0 + wave * 16 + 4 * kq;
+        if constexpr (FUSED) {
+            if (r0 / 2 < nrows) o[r0 / 2] = glu_apply(glu.op, a[0], a[2], glu.alpha, glu.limit);
+            if (r0 / 2 + 1 < nrows) o[r0 / 2 + 1] = glu_apply(glu.op, a[1], a[3], glu.alpha, glu.limit);
+            return;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (r0 + v < nrows) o[r0 + v] = a[v];
+    };
+
     if constexpr (PACK) {
         // the odd sub-blocks' half of each output column (lanes li + 8) onto the even half
 #pragma unroll
         for (int v = 0; v < 4; ++v) acc[0][v] += __shfl_xor(acc[0][v], 8, 64);
         if (li >= 8 || li >= ncols) return;
-        float *o = partial ? partial + ((int64_t)z * ncols + li) * nrows : dst + (int64_t)li * dst_col_stride;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int64_t r = row0 + wave * 16 + 4 * kq + v;
-            if (r < nrows) o[r] = acc[0][v];
-        }
+        store_rows(partial ? partial + ((int64_t)z * ncols + li) * nrows : dst + (int64_t)li * dst_col_stride, acc[0]);
         return;
     }
 #pragma unroll
     for (int j = 0; j < NCT; ++j) {
         const int c = 16 * j + li;
         if (c >= ncols) continue;
-        float *o = partial ? partial + ((int64_t)z * ncols + c) * nrows : dst + (int64_t)c * dst_col_stride;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int64_t r = row0 + wave * 16 + 4 * kq + v;
-            if (r < nrows) o[r] = acc[j][v];
-        }
+        store_rows(partial ? partial + ((int64_t)z * ncols + c) * nrows : dst + (int64_t)c * dst_col_stride, acc[j]);
     }
 }
 
@@ -779,10 +823,11 @@ bool mmq_few_takes(int type, int64_t K, const void *w, int64_t row_stride) {
 // split-K partials when split > 1.
 int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *yqs,
                    const void *yds, int64_t ncols, float *dst, int64_t dst_col_stride, int split, float *partial,
-                   hipStream_t s) {
-    const int64_t gx = (nrows + 16 * FEW_NW - 1) / (16 * FEW_NW);
+                   const MmqGlu &glu, hipStream_t s) {
+    const int64_t gx = ((glu.gate ? 2 * nrows : nrows) + 16 * FEW_NW - 1) / (16 * FEW_NW);
     if (ncols < 1 || ncols > FBN || gx > 0x7FFFFFFF || split < 1 || split > 16 || K / QK_K > 0x7FFFFFFF ||
-        !mmq_few_takes(type, K, w, row_stride))
+        !mmq_few_takes(type, K, w, row_stride) ||
+        (glu.gate && (split != 1 || !mmq_few_takes(type, K, glu.gate, row_stride))))
         return (int)hipErrorInvalidValue;
     const dim3 grid((unsigned)gx, 1, (unsigned)split);
     // two K halves per workgroup where the K parts split evenly
@@ -790,13 +835,15 @@ int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t ro
     const uint8_t *wb = (const uint8_t *)w;
     const uint32_t *ds = (const uint32_t *)yds;
     float *pp = split > 1 ? partial : nullptr;
+    const int kh = khalves ? 2 : 1;
+#define FEW_LAUNCH_K(TYPE, NCT, PK, KH, FU)                                                                            \
+    hipLaunchKernelGGL((mmq_few_kernel<TYPE, FEW_NST, FEW_NW, NCT, PK, KH, FU>), grid, dim3(64 * kh * FEW_NW), 0, s,   \
+                       wb, K, nrows, row_stride, yqs, ds, (int)ncols, dst, dst_col_stride, pp, glu)
 #define FEW_LAUNCH_P(TYPE, NCT, PK)                                                                                    \
-    if (khalves)                                                                                                       \
-        hipLaunchKernelGGL((mmq_few_kernel<TYPE, FEW_NST, FEW_NW, NCT, PK, 2>), grid, dim3(128 * FEW_NW), 0, s, wb, K, \
-                           nrows, row_stride, yqs, ds, (int)ncols, dst, dst_col_stride, pp);                           \
-    else                                                                                                               \
-        hipLaunchKernelGGL((mmq_few_kernel<TYPE, FEW_NST, FEW_NW, NCT, PK, 1>), grid, dim3(64 * FEW_NW), 0, s, wb, K,  \
-                           nrows, row_stride, yqs, ds, (int)ncols, dst, dst_col_stride, pp)
+    if (glu.gate && khalves) FEW_LAUNCH_K(TYPE, NCT, PK, 2, true);                                                     \
+    else if (glu.gate) FEW_LAUNCH_K(TYPE, NCT, PK, 1, true);                                                           \
+    else if (khalves) FEW_LAUNCH_K(TYPE, NCT, PK, 2, false);                                                           \
+    else FEW_LAUNCH_K(TYPE, NCT, PK, 1, false)
 #define FEW_LAUNCH(TYPE, NCT) FEW_LAUNCH_P(TYPE, NCT, false)
     // up to 8 columns of the K-quant nibble types: two sub-blocks per MFMA
     const bool pack = ncols <= FEW_PACK_COLS;
@@ -831,5 +878,6 @@ int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t ro
     }
 #undef FEW_LAUNCH
 #undef FEW_LAUNCH_P
+#undef FEW_LAUNCH_K
     return (int)hipGetLastError();
 }
