@@ -348,7 +348,9 @@ size_t hip_qmm_mmq_workspace_size(int type, int64_t K, int64_t nrows, int64_t nc
  * at most 16 K-steps where 64-column tiles would number at most 256 and
  * 32-column ones at most 512; hip_qmm_mmq_glu does the same over its tiles of
  * 64 output rows, except for Q8_0.  hip_qmm_mmq_split_k: the K-split factor
- * hip_qmm_mmq picks (1: no split; otherwise a divisor of K / 256). */
+ * hip_qmm_mmq picks (1: no split; otherwise a divisor of K / 256); up to 32
+ * columns, matrices of at most 12224 rows and 64 Mi weights run all their
+ * K parts inside one workgroup instead and leave the workspace alone. */
 int hip_qmm_mmq_tile_n(int64_t ncols);
 int hip_qmm_mmq_split_k(int type, int64_t K, int64_t nrows, int64_t ncols);
 

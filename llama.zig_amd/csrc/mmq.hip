@@ -59,6 +59,7 @@ int mmq_q5k_dma_launch(int bn, const void *w, int64_t K, int64_t nrows, int64_t 
                        const qmm_dma::MmqGroups *grp, const MmqGlu &glu, hipStream_t s);
 // mmq_few.hip: the Q4_K / Q8_0 / Q6_K kernel for at most 32 columns
 int mmq_few_split_k(int64_t K, int64_t nrows);
+bool mmq_few_whole_k(int64_t K, int64_t nrows);
 bool mmq_few_takes(int type, int64_t K, const void *w, int64_t row_stride);
 int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *yqs,
                    const void *yds, int64_t ncols, float *dst, int64_t dst_col_stride, int split, float *partial,
@@ -937,7 +938,7 @@ extern "C" int hip_qmm_mmq(int type, const void *w, int64_t K, int64_t nrows, in
     const bool few = few_cols_type(type, K, nrows, ncols) && mmq_few_takes(type, K, w, row_stride) &&
                      (uintptr_t)y_qs % 16 == 0 && (uintptr_t)y_ds % 16 == 0;
     // split K only when the caller's workspace holds the partials
-    int split = few ? mmq_few_split_k(K, nrows) : split_std(type, K, nrows, ncols);
+    int split = !few ? split_std(type, K, nrows, ncols) : mmq_few_whole_k(K, nrows) ? 1 : mmq_few_split_k(K, nrows);
     if (split > 1 && (!workspace || workspace_size < (size_t)split * (size_t)nrows * (size_t)ncols * sizeof(float) ||
                       (uintptr_t)workspace % 16))
         split = 1;

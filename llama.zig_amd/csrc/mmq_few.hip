@@ -18,8 +18,8 @@
 // high) and all <= 32 columns (one or two 16-column tiles), over its share of
 // the K-steps (split K over grid z when the row tiles alone do not fill the
 // chip).  Each K-step (one Q4_K super-block) moves from global memory straight
-// into LDS with global_load_lds_dwordx4, in 1 KiB transfers (14 per step with
-// one column tile, 18 with two):
+// into LDS with global_load_lds_dwordx4, in 1 KiB transfers (12 per step up to
+// 8 columns, 14 with one column tile, 18 with two):
 //   - A: the 64 rows' 144-byte blocks as stored (contiguous 144-byte runs);
 //   - B: the columns' 256 Q8_1 codes, 16-byte chunk c of column n at position
 //     c ^ n, so the operand reads of 16 columns spread over the banks;
@@ -28,6 +28,12 @@
 // are in flight, and a wave waits only for its own transfers of step k
 // (vmcnt = its transfer count of one step) before the step's barrier.  The
 // weight decode (nibbles, scales) is shared by the column tiles.
+//
+// Below 192 such row tiles (and 64 Mi weights) the grid is of 16-row workgroups
+// instead, whose 8 waves each own a share of K and a stage of their own
+// (mmq_few_whole_k): the split's partials and their second launch of ~2-4 us
+// are gone.  4096x4096 at 13 columns 8.8 -> 5.3 us, of which ~1.7 is the launch
+// and the rest two dependent step latencies a wave, not bandwidth (9.4 MB).
 //
 // Q5_K (176-byte blocks, 16-byte aligned like Q4_K) takes the Q4_K path with
 // the fifth bit of each element merged from qh (bit g of qh[l] for element l
@@ -115,15 +121,15 @@ struct FewFmt<TYPE_Q6_K> {
 // Workgroup geometry for NW waves of 16 rows each and NCT tiles of 16
 // columns: the step's LDS stage and its 1 KiB transfers (transfer q goes to
 // wave q % NW).
-template <int TYPE, int NW, int NCT>
+template <int TYPE, int NW, int NCT, bool PACK>
 struct FewGeo {
     static constexpr int WROW = FewFmt<TYPE>::WROW;
     static constexpr int BM = 16 * NW;                 // rows per workgroup
     static constexpr int NT = 64 * NW;                 // threads
     static constexpr int A = BM * WROW;                // weights per step
-    static_assert(A % 1024 == 0, "whole weight transfers");
-    static constexpr int B = 16 * NCT * QK_K;          // codes per step
-    static constexpr int D = 16 * NCT * 8 * 4;         // headers per step
+    static constexpr int NC = PACK ? 8 : 16 * NCT;     // columns moved
+    static constexpr int B = NC * QK_K;                // codes per step
+    static constexpr int D = NC * 8 * 4;               // headers per step
     static constexpr int NQ = (A + B + D + 1023) / 1024;
     static constexpr int STAGE = NQ * 1024;
     static constexpr int PER = (NQ + NW - 1) / NW;     // most transfers of one wave
@@ -214,44 +220,53 @@ __device__ __forceinline__ void wait_step(bool big, int ahead) {
 }
 
 // workgroups per CU that the LDS (160 KiB) holds with KH NST-stage rings
-template <int TYPE, int NW, int NCT>
-constexpr int few_occupancy(int nst, int kh = 1) { return 163840 / (kh * nst * FewGeo<TYPE, NW, NCT>::STAGE); }
+template <int TYPE, int NW, int NCT, bool PACK>
+constexpr int few_occupancy(int nst, int kh = 1) {
+    return 163840 / (kh * nst * FewGeo<TYPE, NW, NCT, PACK>::STAGE + 16);
+}
 
-// KH K halves: the workgroup's waves are KH groups of NW, each with its own
-// ring over an equal share of the workgroup's K-steps (the launcher makes the
-// step count a multiple of KH), so two waves with independent work share a
-// SIMD; the groups meet at every ring barrier (equal step counts) and add
-// their sums through LDS at the end, group 0 first (deterministic).
+// KH K parts: the workgroup's waves are KH groups of NW, each over its share of
+// the workgroup's K-steps; the groups add their sums through LDS at the end,
+// group 0 first (deterministic).
+//   - NW = 4 waves, NST-stage rings (KH 1 or 2; the launcher makes the step count
+//     a multiple of KH, since the groups meet at every ring barrier): two waves
+//     with independent work share a SIMD.
+//   - NW = 1 (NST = 1, KH = 8): each wave fills a stage of its own, contracts it
+//     and fills it again; no barrier until the sums meet, and the other waves of
+//     the CU cover the waits.
 template <int TYPE, int NST, int NW, int NCT, bool PACK, int KH, bool FUSED>
-__global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TYPE, NW, NCT>(NST, KH))) void mmq_few_kernel(
+__global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupancy<TYPE, NW, NCT, PACK>(NST, KH))) void mmq_few_kernel(
     const uint8_t *__restrict__ w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *__restrict__ yqs,
     const uint32_t *__restrict__ yds, int ncols, float *__restrict__ dst, int64_t dst_col_stride,
     float *__restrict__ partial, MmqGlu glu) {
     static_assert(!PACK || (NCT == 1 && (TYPE == TYPE_Q4_K || TYPE == TYPE_Q5_K || TYPE == TYPE_Q6_K)),
                   "packed: one tile, K-quants");
-    using G = FewGeo<TYPE, NW, NCT>;
+    using G = FewGeo<TYPE, NW, NCT, PACK>;
     using FF = FewFmt<TYPE>;
     constexpr int FA = G::A, FB = G::B, FD = G::D, FNQ = G::NQ, PER = G::PER, WROW = G::WROW;
-    constexpr int NQA = FA / 1024;  // transfers 0 .. NQA-1 move weights
-    static_assert(NST >= 2 && few_occupancy<TYPE, NW, NCT>(NST, KH) >= 1, "ring depth");
-    static_assert((NST - 2) * G::transfers_of(0) <= 63, "vmcnt field");
-    static_assert(KH == 1 || NCT * NW * 1024 <= G::STAGE, "K-half sums fit one stage");
+    constexpr int NQA = FA / 1024;             // transfers 0 .. NQA-1 move weights only
+    constexpr bool MIXED = FA % 1024 != 0;     // transfer NQA moves weights and codes
+    constexpr bool PRIVATE = NST == 1;         // one wave, one stage per K part
+    static_assert(PRIVATE == (NW == 1) && few_occupancy<TYPE, NW, NCT, PACK>(NST, KH) >= 1, "ring depth");
+    static_assert(PRIVATE || (NST - 2) * G::transfers_of(0) <= 63, "vmcnt field");
+    static_assert((KH - 1) * NCT * NW * 1024 <= KH * NST * G::STAGE, "the K parts' sums fit the stages");
     __shared__ alignas(16) uint8_t rings[KH][NST][G::STAGE];
     __shared__ alignas(16) uint4 zero16;  // the packed path's B operand for the lanes of the other sub-block
     if (PACK && threadIdx.x == 0) zero16 = make_uint4(0u, 0u, 0u, 0u);  // published by the ring's first barrier
+    if constexpr (PACK && PRIVATE) __syncthreads();                      // (private stages have none)
 
     const int64_t Kp = pad_k(K);
     const int lane = threadIdx.x & 63;
     const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int kh = wave_all / NW, wave = wave_all - kh * NW;  // K half, wave within it
+    const int kh = wave_all / NW, wave = wave_all - kh * NW;  // K part, wave within it
     uint8_t(*st)[G::STAGE] = rings[kh];
     const int li = lane & 15, kq = lane >> 4;
     const int64_t row0 = (int64_t)blockIdx.x * G::BM;  // FUSED: of the gate and up rows together
     const int nkb = (int)(K / QK_K);
     const int gz = (int)gridDim.z, z = (int)blockIdx.z;
     const int kz0 = (int)((int64_t)nkb * z / gz), kz1 = (int)((int64_t)nkb * (z + 1) / gz);
-    const int nkh = (kz1 - kz0) / KH;  // steps per K half (the launcher makes them equal)
-    const int kb0 = kz0 + kh * nkh, kb1 = kb0 + nkh;
+    // this K part's steps (rings: equal counts, by the launcher: they meet at barriers)
+    const int kb0 = kz0 + (kz1 - kz0) * kh / KH, kb1 = kz0 + (kz1 - kz0) * (kh + 1) / KH;
 
     // Per-lane sources of this wave's transfers (q = wave + NW*i), as a base
     // at K-step 0 and the bytes one K-step adds.
@@ -266,7 +281,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
             const int64_t trow = FUSED ? row0 / 2 + mmq_glu_tile_row(r) : row0 + r;
             const int64_t grow = trow < nrows ? trow : nrows - 1;  // rows past the end: duplicates
             src[i] = (FUSED && (r & 2) == 0 ? glu.gate : w) + grow * row_stride + off;
-            kstep[i] = 0;  // the weights' step offset is FF::aoff
+            kstep[i] = -1;  // the weights' step offset is FF::aoff
         } else if (pos < FA + FB) {
             const int p = pos - FA, n = p >> 8, c = ((p >> 4) & 15) ^ (n & 15);
             const int col = n < ncols ? n : ncols - 1;  // columns past the end: duplicates
@@ -286,7 +301,9 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const int q = wave + NW * i;  // uniform
-            if (q < FNQ) dma16(src[i] + (q < NQA ? ao : (int64_t)kb * kstep[i]), st + q * 1024);
+            if (q < NQA) dma16(src[i] + ao, st + q * 1024);
+            else if (MIXED && q == NQA) dma16(src[i] + (kstep[i] < 0 ? ao : (int64_t)kb * kstep[i]), st + q * 1024);
+            else if (q < FNQ) dma16(src[i] + (int64_t)kb * kstep[i], st + q * 1024);
         }
     };
 
@@ -687,26 +704,39 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
         }
     };
 
-    // NST-stage ring: step kb0 + i lives in stage i % NST; while a step is
-    // contracted, the next NST - 2 are in flight and one more is issued
-    const bool big = wave < FNQ % NW || FNQ % NW == 0;
+    auto contract = [&](const uint8_t *stage, int kb) {
+        if constexpr (PACK && TYPE == TYPE_Q6_K) compute_q6_k_pack(stage, kb);
+        else if constexpr (PACK) compute_pack(stage);
+        else if constexpr (TYPE == TYPE_Q4_K || TYPE == TYPE_Q5_K) compute(stage);
+        else if constexpr (TYPE == TYPE_Q8_0 || TYPE == TYPE_Q4_0) compute_q8_0(stage);
+        else if constexpr (TYPE == TYPE_IQ4_XS) compute_iq4_xs(stage, kb);
+        else compute_q6_k(stage, kb);
+    };
+    if constexpr (PRIVATE) {
+        for (int kb = kb0; kb < kb1; ++kb) {
+            dma(kb, st[0]);
+            wait_vm<0>();
+            asm volatile("" ::: "memory");  // the stage's reads stay below the wait,
+            contract(st[0], kb);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and are done before it is refilled
+        }
+    } else {
+        // NST-stage ring: step kb0 + i lives in stage i % NST; while a step is
+        // contracted, the next NST - 2 are in flight and one more is issued
+        const bool big = wave < FNQ % NW || FNQ % NW == 0;
 #pragma unroll
-    for (int i = 0; i < NST - 1; ++i)
-        if (kb0 + i < kb1) dma(kb0 + i, st[i]);
-    for (int kb = kb0; kb < kb1;) {
+        for (int i = 0; i < NST - 1; ++i)
+            if (kb0 + i < kb1) dma(kb0 + i, st[i]);
+        for (int kb = kb0; kb < kb1;) {
 #pragma unroll
-        for (int i = 0; i < NST; ++i) {
-            const int left = kb1 - 1 - kb;  // steps after kb already issued: min(left, NST - 2)
-            wait_step<NST - 2, G::transfers_of(0), G::transfers_of(NW - 1)>(big, left < NST - 2 ? left : NST - 2);
-            lds_barrier();
-            if (kb + NST - 1 < kb1) dma(kb + NST - 1, st[(i + NST - 1) % NST]);
-            if constexpr (PACK && TYPE == TYPE_Q6_K) compute_q6_k_pack(st[i], kb);
-            else if constexpr (PACK) compute_pack(st[i]);
-            else if constexpr (TYPE == TYPE_Q4_K || TYPE == TYPE_Q5_K) compute(st[i]);
-            else if constexpr (TYPE == TYPE_Q8_0 || TYPE == TYPE_Q4_0) compute_q8_0(st[i]);
-            else if constexpr (TYPE == TYPE_IQ4_XS) compute_iq4_xs(st[i], kb);
-            else compute_q6_k(st[i], kb);
-            if (++kb >= kb1) break;
+            for (int i = 0; i < NST; ++i) {
+                const int left = kb1 - 1 - kb;  // steps after kb already issued: min(left, NST - 2)
+                wait_step<NST - 2, G::transfers_of(0), G::transfers_of(NW - 1)>(big, left < NST - 2 ? left : NST - 2);
+                lds_barrier();
+                if (kb + NST - 1 < kb1) dma(kb + NST - 1, st[(i + NST - 1) % NST]);
+                contract(st[i], kb);
+                if (++kb >= kb1) break;
+            }
         }
     }
     if constexpr (FUSED) {
@@ -714,18 +744,21 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT>::NT), (few_occupancy<TY
         for (int j = 0; j < NCT; ++j) acc[j] += lost[j];
     }
     if constexpr (KH > 1) {
-        // every wave's ring reads (and transfers: the last wait was vmcnt(0))
-        // are done; K half 1 hands its sums to half 0 through the first stage
+        // every wave's stage reads (and transfers: the last wait was vmcnt(0))
+        // are done; K parts 1.. hand their sums to part 0 through the stages'
+        // memory, which adds them in order
         lds_barrier();
         v4f *part = reinterpret_cast<v4f *>(&rings[0][0][0]);
-        if (kh == 1) {
+        if (kh > 0) {
 #pragma unroll
-            for (int j = 0; j < NCT; ++j) part[(j * NW + wave) * 64 + lane] = acc[j];
+            for (int j = 0; j < NCT; ++j) part[(((kh - 1) * NCT + j) * NW + wave) * 64 + lane] = acc[j];
         }
         lds_barrier();
-        if (kh == 1) return;
+        if (kh > 0) return;
 #pragma unroll
-        for (int j = 0; j < NCT; ++j) acc[j] += part[(j * NW + wave) * 64 + lane];
+        for (int k = 0; k < KH - 1; ++k)
+#pragma unroll
+            for (int j = 0; j < NCT; ++j) acc[j] += part[((k * NCT + j) * NW + wave) * 64 + lane];
     }
 
     // a lane's four rows of a column; fused, gate (v = 0, 1) and up (v = 2, 3) of two output rows
@@ -786,6 +819,26 @@ int mmq_few_split_k(int64_t K, int64_t nrows) {
     return (int)split;
 }
 
+// Whether 16-row workgroups of 8 waves, one K part each, take the launch
+// (NST = 1, NW = 1): all of K inside one workgroup, so no partials and no second
+// launch to add them, and 4 times the workgroups.  Their 16 rows share the
+// columns' codes among 16 rows instead of 64, so the codes are most of what moves
+// into LDS and the 64-row tiles stay ahead on unsplit grids (>= 192 of them) and
+// where the weights stream long enough to hide the reduction.  Graph-timed,
+// kernel (+ reduction), 64-row tiles -> these, us at 13 columns unless given:
+//   Q4_K 4096x4096 at 4 / 13 / 32: 8.0 / 8.8 / 11.5 -> 5.5 / 5.3 / 7.0
+//   Q4_K 1024x4096 7.1 -> 4.7, 333x4096 9.7 -> 4.2, 256x256 3.2 -> 3.1
+//   Q4_K 4096x14336 at 4 / 13 / 24: 13.8 / 14.6 / 19.7 -> 11.8 / 13.0 / 18.0
+//   Q5_K 4096x14336 15.9 -> 14.1, Q6_K 24.8 -> 21.8 (at 4: 20.1 -> 15.3),
+//   Q8_0 18.7 -> 17.1, IQ4_XS 17.3 -> 13.9
+//   Q4_K 6144x4096 10.3 -> 7.1, 10240x4096 13.5 -> 11.5, 8192x8192 15.5 -> 14.7,
+//   10240x8192 19.3 -> 19.4, 8192x28672 37.1 -> 42.0; unsplit 14336x4096 12.3 -> 14.4
+// 1 stage and 8 parts: of 1-2 stages and 3-16 parts the best or within 5% on every
+// shape (4 parts of 2 stages 10240x4096 12.1, 16 of 1 stage 14.0; two stages of 8
+// gain 2% on 14336 at 4 columns and lose 25% on 6144 rows).
+constexpr int FEW_PARTS = 8;
+bool mmq_few_whole_k(int64_t K, int64_t nrows) { return nrows <= 191 * 16 * FEW_NW && nrows * K <= ((int64_t)64 << 20); }
+
 // Whether a workgroup runs two K halves of its K part (KH = 2): K parts of
 // an even step count, at least 4, on grids of at most 256 workgroups (two
 // rings take twice the LDS, so a workgroup fills a CU's LDS by itself: a
@@ -824,10 +877,12 @@ bool mmq_few_takes(int type, int64_t K, const void *w, int64_t row_stride) {
 int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *yqs,
                    const void *yds, int64_t ncols, float *dst, int64_t dst_col_stride, int split, float *partial,
                    const MmqGlu &glu, hipStream_t s) {
-    const int64_t gx = ((glu.gate ? 2 * nrows : nrows) + 16 * FEW_NW - 1) / (16 * FEW_NW);
+    const bool whole_k = !glu.gate && mmq_few_whole_k(K, nrows);
+    const int64_t bm = whole_k ? 16 : 16 * FEW_NW;
+    const int64_t gx = ((glu.gate ? 2 * nrows : nrows) + bm - 1) / bm;
     if (ncols < 1 || ncols > FBN || gx > 0x7FFFFFFF || split < 1 || split > 16 || K / QK_K > 0x7FFFFFFF ||
         !mmq_few_takes(type, K, w, row_stride) ||
-        (glu.gate && (split != 1 || !mmq_few_takes(type, K, glu.gate, row_stride))))
+        ((glu.gate || whole_k) && split != 1) || (glu.gate && !mmq_few_takes(type, K, glu.gate, row_stride)))
         return (int)hipErrorInvalidValue;
     const dim3 grid((unsigned)gx, 1, (unsigned)split);
     // two K halves per workgroup where the K parts split evenly
@@ -835,15 +890,15 @@ int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t ro
     const uint8_t *wb = (const uint8_t *)w;
     const uint32_t *ds = (const uint32_t *)yds;
     float *pp = split > 1 ? partial : nullptr;
-    const int kh = khalves ? 2 : 1;
-#define FEW_LAUNCH_K(TYPE, NCT, PK, KH, FU)                                                                            \
-    hipLaunchKernelGGL((mmq_few_kernel<TYPE, FEW_NST, FEW_NW, NCT, PK, KH, FU>), grid, dim3(64 * kh * FEW_NW), 0, s,   \
-                       wb, K, nrows, row_stride, yqs, ds, (int)ncols, dst, dst_col_stride, pp, glu)
+#define FEW_LAUNCH_K(TYPE, NST, NW, NCT, PK, KH, FU)                                                                   \
+    hipLaunchKernelGGL((mmq_few_kernel<TYPE, NST, NW, NCT, PK, KH, FU>), grid, dim3(64 * NW * KH), 0, s, wb, K, nrows, \
+                       row_stride, yqs, ds, (int)ncols, dst, dst_col_stride, pp, glu)
 #define FEW_LAUNCH_P(TYPE, NCT, PK)                                                                                    \
-    if (glu.gate && khalves) FEW_LAUNCH_K(TYPE, NCT, PK, 2, true);                                                     \
-    else if (glu.gate) FEW_LAUNCH_K(TYPE, NCT, PK, 1, true);                                                           \
-    else if (khalves) FEW_LAUNCH_K(TYPE, NCT, PK, 2, false);                                                           \
-    else FEW_LAUNCH_K(TYPE, NCT, PK, 1, false)
+    if (whole_k) FEW_LAUNCH_K(TYPE, 1, 1, NCT, PK, FEW_PARTS, false);                                                  \
+    else if (glu.gate && khalves) FEW_LAUNCH_K(TYPE, FEW_NST, FEW_NW, NCT, PK, 2, true);                               \
+    else if (glu.gate) FEW_LAUNCH_K(TYPE, FEW_NST, FEW_NW, NCT, PK, 1, true);                                          \
+    else if (khalves) FEW_LAUNCH_K(TYPE, FEW_NST, FEW_NW, NCT, PK, 2, false);                                          \
+    else FEW_LAUNCH_K(TYPE, FEW_NST, FEW_NW, NCT, PK, 1, false)
 #define FEW_LAUNCH(TYPE, NCT) FEW_LAUNCH_P(TYPE, NCT, false)
     // up to 8 columns of the K-quant nibble types: two sub-blocks per MFMA
     const bool pack = ncols <= FEW_PACK_COLS;
