@@ -86,7 +86,9 @@ size_t hip_qmm_mul_mat_glu_workspace_preferred(int type, int64_t K, int64_t nrow
 
 /* 1 if hip_qmm_mul_mat runs an MMQ kernel (the few-column GEMM or the tile)
  * rather than the GEMV for this shape on 16-byte-aligned rows, else 0 (the
- * shape rules that hip_qmm_mul_mat_workspace_size applies).  No counterpart
+ * shape rules that hip_qmm_mul_mat_workspace_size applies; 3-8 columns of
+ * 2048-12224 rows also run the few-column GEMM's form that needs no workspace
+ * beyond the Q8_1 planes where that is faster, with 0 here).  No counterpart
  * in the reference: a query for measurement and tests that time or check the
  * kernel the op takes. */
 int hip_qmm_mul_mat_uses_mmq(int type, int64_t K, int64_t nrows, int64_t ncols);
@@ -288,12 +290,13 @@ int hip_qmm_gemv_mfma(int type, const void *w, int64_t K, int64_t nrows, int64_t
  *    (hip_qmm_mul_mat_per_column), with no workspace;
  *  - the few-column GEMM (16x16 int8 MFMA tiles) for 9-32 columns (9-16 for
  *    Q6_K; Q8_0 / Q4_0 at 17-32 columns of 8 MiB of weights and more take the
- *    tile), and also for 4-8 columns of large matrices, where it measured
+ *    tile above K = 4096 or 16 Mi weights), and also for 4-8 columns of large matrices, where it measured
  *    faster than the GEMV (the shape rules are hip_qmm_mul_mat_workspace_size's
  *    and hip_qmm_mul_mat_uses_mmq's: e.g. Q4_K from 5 columns at K >= 8192 on
  *    >= 4096 rows and on >= 12288 rows, from 7 columns on >= 6144 rows; Q6_K
- *    from 4 columns on >= 24M weights of long rows or >= 12288 rows).  On
- *    those 4-8 column shapes the workspace grows by the
+ *    from 4 columns on >= 24M weights of long rows or >= 12288 rows; and 3-8
+ *    columns of 2048-12224 rows where its form without partials wins).  On
+ *    the shapes that hip_qmm_mul_mat_uses_mmq reports the workspace grows by the
  *    few-column kernel's split-K partials, and the results differ from
  *    hip_qmm_mul_mat_vec's in fp32 rounding (another summation order; both
  *    pass the f64 and CPU gates);
@@ -349,7 +352,7 @@ size_t hip_qmm_mmq_workspace_size(int type, int64_t K, int64_t nrows, int64_t nc
  * 32-column ones at most 512; hip_qmm_mmq_glu does the same over its tiles of
  * 64 output rows, except for Q8_0.  hip_qmm_mmq_split_k: the K-split factor
  * hip_qmm_mmq picks (1: no split; otherwise a divisor of K / 256); up to 32
- * columns, matrices of at most 12224 rows and 64 Mi weights run all their
+ * columns, most matrices of at most 12224 rows and 64 Mi weights run all their
  * K parts inside one workgroup instead and leave the workspace alone. */
 int hip_qmm_mmq_tile_n(int64_t ncols);
 int hip_qmm_mmq_split_k(int type, int64_t K, int64_t nrows, int64_t ncols);

@@ -20,6 +20,7 @@ extern "C" size_t hip_qmm_mmq_workspace_size(int type, int64_t K, int64_t nrows,
 bool few_cols_type(int type, int64_t K, int64_t nrows, int64_t ncols);
 // mmq_few.hip: whether it takes these weight rows
 bool mmq_few_takes(int type, int64_t K, const void *w, int64_t row_stride);
+bool mmq_few_whole_k(int type, int64_t K, int64_t nrows, int64_t ncols);
 
 int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *yqs,
                    const void *yds, int64_t ncols, float *dst, int64_t dst_col_stride, int split, float *partial,
@@ -121,6 +122,37 @@ bool few_cols_wins(int type, int64_t K, int64_t nrows, int64_t ncols) {
     }
 }
 
+// Whether 3-8 columns go to the few-column kernel beyond few_cols_wins because its
+// 16-row workgroups hold all of K there (mmq_few_whole_k): one launch after the
+// quantizer and no partials, so the workspace needs nothing beyond the Q8_1 planes
+// and hip_qmm_mul_mat_uses_mmq (which sizes for partials) does not report it.  The
+// least columns at which quantizer + GEMM is ahead of the GEMV, by rows and K, from
+// graph-timed calls (GEMV -> few, us): Q4_K 4096x4096 at 5 / 6 / 8 7.6 -> 7.4, 8.9 ->
+// 7.4, 9.5 -> 7.4 (at 4 6.9 / 7.3), 6144x2048 at 3 7.3 -> 6.8, 2048x4096 at 7 8.0 ->
+// 7.1; rows below 2048 keep the GEMV (1024x4096 at 8 5.3 / 6.9), and so do the shapes
+// of hip_qmm_mul_mat_per_column and, on at most 4096 rows and K, the columns that one
+// launch of the quantize-in-GEMV kernel takes: their results are the one-column
+// kernel's.
+bool few_whole_wins(int type, int64_t K, int64_t nrows, int64_t ncols) {
+    if (K % 256 != 0 || ncols < 3 || ncols > 8 || nrows < 2048 || !few_cols_type(type, K, nrows, ncols) ||
+        !mmq_few_whole_k(type, K, nrows, ncols) || hip_qmm_mul_mat_per_column(type, K, nrows, ncols))
+        return false;
+    if (nrows <= 4096 && K <= 4096 && ncols <= (type == TYPE_Q8_0 ? 8 : type == TYPE_IQ4_XS ? 6 : 4)) return false;
+    //                          K < 4096, K < 8192, more
+    static constexpr int8_t least[6][3][3] = {
+        // rows from 2048   4096         6144
+        {{9, 7, 6}, {5, 6, 4}, {3, 5, 4}},  // Q4_K
+        {{9, 5, 5}, {4, 5, 4}, {4, 5, 4}},  // Q5_K
+        {{9, 5, 5}, {5, 5, 4}, {4, 4, 4}},  // Q6_K
+        {{9, 9, 5}, {5, 5, 4}, {5, 5, 4}},  // Q8_0
+        {{9, 6, 5}, {8, 6, 5}, {8, 8, 5}},  // Q4_0
+        {{9, 6, 6}, {6, 6, 5}, {6, 7, 5}},  // IQ4_XS
+    };
+    const int t = type == TYPE_Q4_K ? 0 : type == TYPE_Q5_K ? 1 : type == TYPE_Q6_K ? 2 : type == TYPE_Q8_0 ? 3
+                : type == TYPE_Q4_0 ? 4 : 5;
+    return ncols >= least[t][nrows >= 6144 ? 2 : nrows >= 4096 ? 1 : 0][K >= 8192 ? 2 : K >= 4096 ? 1 : 0];
+}
+
 // Shape-only (the workspace sizing): the MMQ dispatch takes these columns.
 bool use_mmq(int type, int64_t K, int64_t nrows, int64_t ncols) {
     return K % 256 == 0 && (ncols > 8 || few_cols_wins(type, K, nrows, ncols));
@@ -130,7 +162,8 @@ bool use_mmq(int type, int64_t K, int64_t nrows, int64_t ncols) {
 // the rows (16-byte-aligned rows for the 2- and 8-byte-aligned types); the
 // MMQ tile would be slower than the GEMV there.
 bool use_mmq_rows(int type, int64_t K, int64_t nrows, int64_t ncols, const void *w, int64_t row_stride) {
-    return use_mmq(type, K, nrows, ncols) && (ncols > 8 || mmq_few_takes(type, K, w, row_stride));
+    return (use_mmq(type, K, nrows, ncols) || few_whole_wins(type, K, nrows, ncols)) &&
+           (ncols > 8 || mmq_few_takes(type, K, w, row_stride));
 }
 
 // Whether gate/up/GLU over ncols columns runs the fused MMQ: where each

@@ -59,7 +59,7 @@ int mmq_q5k_dma_launch(int bn, const void *w, int64_t K, int64_t nrows, int64_t 
                        const qmm_dma::MmqGroups *grp, const MmqGlu &glu, hipStream_t s);
 // mmq_few.hip: the Q4_K / Q8_0 / Q6_K kernel for at most 32 columns
 int mmq_few_split_k(int64_t K, int64_t nrows);
-bool mmq_few_whole_k(int64_t K, int64_t nrows);
+bool mmq_few_whole_k(int type, int64_t K, int64_t nrows, int64_t ncols);
 bool mmq_few_takes(int type, int64_t K, const void *w, int64_t row_stride);
 int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *yqs,
                    const void *yds, int64_t ncols, float *dst, int64_t dst_col_stride, int split, float *partial,
@@ -905,6 +905,17 @@ bool few_cols_type(int type, int64_t K, int64_t nrows, int64_t ncols) {
     return true;
 }
 
+// Q8_0 and Q4_0 at 17-32 columns of 8 MiB and more take the few-column kernel after
+// all where its workgroups hold all of K, up to K = 4096 and 16 Mi weights (whole
+// call, tile -> few, us, at 24 columns: Q8_0 4096x4096 14.9 -> 11.7, 4096x2048 11.5 ->
+// 8.1, 6144x2048 12.3 -> 11.6; Q4_0 4096x4096 13.6 -> 10.0, 8192x2048 13.9 -> 11.9);
+// above, the tile: Q8_0 2048x8192 15.2 / 15.6, 10240x4096 22.2 / 24.1.  Without
+// partials: the split and workspace queries keep the tile's answers.
+static bool few_wide(int type, int64_t K, int64_t nrows, int64_t ncols) {
+    return (type == TYPE_Q8_0 || type == TYPE_Q4_0) && ncols > 16 && ncols <= 32 && K <= 4096 &&
+           nrows * K <= ((int64_t)16 << 20) && mmq_few_whole_k(type, K, nrows, ncols);
+}
+
 // For api.hip's f16 route: the weight checks of this dispatch, and the sum of K-split partials.
 int mmq_check_weights(int type, const void *w, int64_t K, int64_t row_stride) {
     return check_weights(type, w, K, row_stride);
@@ -935,10 +946,11 @@ extern "C" int hip_qmm_mmq(int type, const void *w, int64_t K, int64_t nrows, in
     if (int e = check_weights(type, w, K, row_stride)) return e;
     const int bn = mmq_bn(type, K, nrows, ncols);
     const int64_t gy = (ncols + bn - 1) / bn;
-    const bool few = few_cols_type(type, K, nrows, ncols) && mmq_few_takes(type, K, w, row_stride) &&
-                     (uintptr_t)y_qs % 16 == 0 && (uintptr_t)y_ds % 16 == 0;
+    const bool few_rows = mmq_few_takes(type, K, w, row_stride) && (uintptr_t)y_qs % 16 == 0 && (uintptr_t)y_ds % 16 == 0;
+    const bool few = few_rows && (few_cols_type(type, K, nrows, ncols) || few_wide(type, K, nrows, ncols));
+    const bool whole_k = few && mmq_few_whole_k(type, K, nrows, ncols);
     // split K only when the caller's workspace holds the partials
-    int split = !few ? split_std(type, K, nrows, ncols) : mmq_few_whole_k(K, nrows) ? 1 : mmq_few_split_k(K, nrows);
+    int split = !few ? split_std(type, K, nrows, ncols) : whole_k ? 1 : mmq_few_split_k(K, nrows);
     if (split > 1 && (!workspace || workspace_size < (size_t)split * (size_t)nrows * (size_t)ncols * sizeof(float) ||
                       (uintptr_t)workspace % 16))
         split = 1;

@@ -281,7 +281,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupa
             const int64_t trow = FUSED ? row0 / 2 + mmq_glu_tile_row(r) : row0 + r;
             const int64_t grow = trow < nrows ? trow : nrows - 1;  // rows past the end: duplicates
             src[i] = (FUSED && (r & 2) == 0 ? glu.gate : w) + grow * row_stride + off;
-            kstep[i] = -1;  // the weights' step offset is FF::aoff
+            kstep[i] = MIXED ? -1 : 0;  // the weights' step offset is FF::aoff
         } else if (pos < FA + FB) {
             const int p = pos - FA, n = p >> 8, c = ((p >> 4) & 15) ^ (n & 15);
             const int col = n < ncols ? n : ncols - 1;  // columns past the end: duplicates
@@ -301,9 +301,8 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupa
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const int q = wave + NW * i;  // uniform
-            if (q < NQA) dma16(src[i] + ao, st + q * 1024);
-            else if (MIXED && q == NQA) dma16(src[i] + (kstep[i] < 0 ? ao : (int64_t)kb * kstep[i]), st + q * 1024);
-            else if (q < FNQ) dma16(src[i] + (int64_t)kb * kstep[i], st + q * 1024);
+            const bool weights = q < NQA || (MIXED && kstep[i] < 0);
+            if (q < FNQ) dma16(src[i] + (weights ? ao : (int64_t)kb * kstep[i]), st + q * 1024);
         }
     };
 
@@ -836,8 +835,33 @@ int mmq_few_split_k(int64_t K, int64_t nrows) {
 // 1 stage and 8 parts: of 1-2 stages and 3-16 parts the best or within 5% on every
 // shape (4 parts of 2 stages 10240x4096 12.1, 16 of 1 stage 14.0; two stages of 8
 // gain 2% on 14336 at 4 columns and lose 25% on 6144 rows).
+//
+// Where a workgroup's steps are many and its rows few, a wave's steps one after the
+// other outlast the split's shorter shares and second launch, so the rows have to
+// grow with the steps of a part; steps with more work (Q6_K, two column tiles) reach
+// that point earlier.  Whole call, split -> whole K, us: Q4_K 2048 / 1024 / 512 x
+// 14336 at 13 13.6 -> 12.8, 11.7 -> 11.0, 11.0 -> 10.9, IQ4_XS 512 10.9 -> 12.8; Q6_K
+// 2048 / 1024 x 8192 at 13 14.3 -> 13.9, 11.7 -> 13.0, 2048x14336 18.2 -> 19.8; two
+// tiles 1024x14336 at 24 14.0 -> 15.4, 2048x8192 11.9 -> 9.8.  K / 256 without a
+// divisor to split by (K = 11008: 1024 rows ran 31 us unsplit) has no shorter shares.
+//
+// Above 4096 rows a CU takes a second workgroup: the 64-row form stays below 4 steps
+// (11008x512 at 9 6.3 / 8.3), from 40 Mi weights on (Q4_K 7168x8192 at 13 17.4 / 18.0;
+// Q6_K, whose steps hide the transfers, gains to the end: 8192x8192 27 -> 22) and, with
+// two tiles (96 KiB of stages, so rounds of 256), unless at most 8192 rows share out
+// two even steps a part (6144x4096 at 24 12.5 -> 11.2; 5120x3072 13.2 / 13.6, 5120x6144
+// 17.3 / 18.4, 10240x1024 12.1 / 13.1).
 constexpr int FEW_PARTS = 8;
-bool mmq_few_whole_k(int64_t K, int64_t nrows) { return nrows <= 191 * 16 * FEW_NW && nrows * K <= ((int64_t)64 << 20); }
+bool mmq_few_whole_k(int type, int64_t K, int64_t nrows, int64_t ncols) {
+    if (nrows > 191 * 16 * FEW_NW || nrows * K > ((int64_t)64 << 20)) return false;
+    const int64_t nkb = K / QK_K, steps = (nkb + FEW_PARTS - 1) / FEW_PARTS;
+    if (nrows > 4096) {
+        if (nkb < 4 || (type != TYPE_Q6_K && nrows * K >= ((int64_t)40 << 20))) return false;
+        if (ncols > 16 && (nrows > 8192 || nkb % FEW_PARTS != 0 || steps > 2)) return false;
+    }
+    const bool heavy = type == TYPE_Q6_K || ncols > 16;
+    return steps <= (heavy ? 2 : 4) || nrows >= (heavy ? 512 : 256) * steps || nkb / mmq_few_split_k(K, nrows) >= steps;
+}
 
 // Whether a workgroup runs two K halves of its K part (KH = 2): K parts of
 // an even step count, at least 4, on grids of at most 256 workgroups (two
@@ -877,7 +901,7 @@ bool mmq_few_takes(int type, int64_t K, const void *w, int64_t row_stride) {
 int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *yqs,
                    const void *yds, int64_t ncols, float *dst, int64_t dst_col_stride, int split, float *partial,
                    const MmqGlu &glu, hipStream_t s) {
-    const bool whole_k = !glu.gate && mmq_few_whole_k(K, nrows);
+    const bool whole_k = !glu.gate && mmq_few_whole_k(type, K, nrows, ncols);
     const int64_t bm = whole_k ? 16 : 16 * FEW_NW;
     const int64_t gx = ((glu.gate ? 2 * nrows : nrows) + bm - 1) / bm;
     if (ncols < 1 || ncols > FBN || gx > 0x7FFFFFFF || split < 1 || split > 16 || K / QK_K > 0x7FFFFFFF ||

@@ -54,3 +54,39 @@ def test_few_row_limit(nrows, ncols):
     got = G.mmq("Q5_K", w_d, K, qs, ds).cpu().numpy()
     ideal = O.mul_mat_q8_1_f64(O.TYPE_Q5_K, wq, nrows, K, G.quantize_q8_1(x_d, K).cpu().numpy(), ncols)
     assert max_err_scaled(got, ideal) < F64_TOL, max_err_scaled(got, ideal)
+
+
+def _op(G, tname, w_d, K, x_d):
+    """hip_qmm_mul_mat with exactly the workspace that it asks for."""
+    import ctypes
+    ncols, nrows = x_d.shape[0], w_d.shape[0]
+    out = torch.full((ncols, nrows + 3), float("nan"), device="cuda")
+    ws = torch.empty(G.workspace_size(tname, K, ncols, nrows), dtype=torch.uint8, device="cuda")
+    e = G.lib().hip_qmm_mul_mat(TYPES[tname], G._ptr(w_d), K, nrows, w_d.stride(0), G._ptr(x_d), ncols, x_d.stride(0),
+                                G._ptr(out), nrows + 3, G._ptr(ws), ctypes.c_size_t(ws.numel()), G._stream())
+    assert e == 0, e
+    assert np.isnan(out[:, nrows:].cpu().numpy()).all()
+    return out[:, :nrows].cpu().numpy()
+
+
+# 3-8 columns: the least count that each row and K band sends to the few-column GEMM, and one
+# fewer or the GEMV's shapes beside them
+@pytest.mark.parametrize("tname,nrows,K,ncols,few", [
+    ("Q4_K", 6144, 1024, 3, 1), ("Q4_K", 4097, 1024, 5, 1), ("Q4_K", 4097, 1024, 4, 0), ("Q4_K", 2049, 4096, 7, 1),
+    ("Q4_K", 2048, 4096, 7, 0), ("Q5_K", 4097, 1024, 4, 1), ("Q5_K", 4097, 768, 8, 0), ("Q5_K", 4096, 1024, 4, 0), ("Q5_K", 4096, 1024, 5, 1), ("Q5_K", 2050, 8192, 5, 1), ("Q5_K", 2050, 2048, 8, 0),
+    ("Q6_K", 6150, 2048, 4, 1), ("Q6_K", 2050, 4096, 5, 1), ("Q8_0", 4100, 1024, 5, 1), ("Q8_0", 4100, 1024, 4, 0),
+    ("Q4_0", 6144, 1024, 8, 1), ("Q4_0", 6144, 1024, 7, 0), ("IQ4_XS", 4100, 1024, 6, 1), ("IQ4_XS", 2050, 4096, 7, 1),
+    ("Q8_0", 4100, 2048, 17, 1), ("Q4_0", 4100, 4096, 24, 0), ("Q8_0", 4096, 4096, 32, 1),  # whole K, the tile
+])
+def test_op_route(tname, nrows, K, ncols, few):
+    import ggml_hip as G
+    t = TYPES[tname]
+    wq = weights_q(t, nrows, K)
+    w_d = torch.from_numpy(np.array(wq)).cuda()
+    x_d = torch.from_numpy(np.array(acts(ncols, K))).cuda()
+    got = _op(G, tname, w_d, K, x_d)
+    qs, ds = G.quantize_q8_1_planar(x_d)
+    gemm = G.mmq(tname, w_d, K, qs, ds).cpu().numpy()
+    assert np.array_equal(got, gemm) == bool(few or ncols > 8)
+    ideal = O.mul_mat_q8_1_f64(t, wq, nrows, K, G.quantize_q8_1(x_d, K).cpu().numpy(), ncols)
+    assert max_err_scaled(got, ideal) < F64_TOL, max_err_scaled(got, ideal)
