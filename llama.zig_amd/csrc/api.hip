@@ -129,7 +129,8 @@ bool few_cols_wins(int type, int64_t K, int64_t nrows, int64_t ncols) {
 // least columns at which quantizer + GEMM is ahead of the GEMV, by rows and K, from
 // graph-timed calls (GEMV -> few, us): Q4_K 4096x4096 at 5 / 6 / 8 7.6 -> 7.4, 8.9 ->
 // 7.4, 9.5 -> 7.4 (at 4 6.9 / 7.3), 6144x2048 at 3 7.3 -> 6.8, 2048x4096 at 7 8.0 ->
-// 7.1; rows below 2048 keep the GEMV (1024x4096 at 8 5.3 / 6.9), and so do the shapes
+// 7.1; rows below 2048 keep the GEMV (1024x4096 at 8 5.3 / 6.9; Q4_0
+// 2048x8192 at 6 10.3 / 10.9), and so do the shapes
 // of hip_qmm_mul_mat_per_column and, on at most 4096 rows and K, the columns that one
 // launch of the quantize-in-GEMV kernel takes: their results are the one-column
 // kernel's.
@@ -145,7 +146,7 @@ bool few_whole_wins(int type, int64_t K, int64_t nrows, int64_t ncols) {
         {{9, 5, 5}, {4, 5, 4}, {4, 5, 4}},  // Q5_K
         {{9, 5, 5}, {5, 5, 4}, {4, 4, 4}},  // Q6_K
         {{9, 9, 5}, {5, 5, 4}, {5, 5, 4}},  // Q8_0
-        {{9, 6, 5}, {8, 6, 5}, {8, 8, 5}},  // Q4_0
+        {{9, 7, 7}, {8, 7, 5}, {8, 8, 5}},  // Q4_0
         {{9, 6, 6}, {6, 6, 5}, {6, 7, 5}},  // IQ4_XS
     };
     const int t = type == TYPE_Q4_K ? 0 : type == TYPE_Q5_K ? 1 : type == TYPE_Q6_K ? 2 : type == TYPE_Q8_0 ? 3

@@ -32,7 +32,7 @@
 // Below 192 such row tiles (and 64 Mi weights) the grid is of 16-row workgroups
 // instead, whose 8 waves each own a share of K and a stage of their own
 // (mmq_few_whole_k): the split's partials and their second launch of ~2-4 us
-// are gone.  4096x4096 at 13 columns 8.8 -> 5.3 us, of which ~1.7 is the launch
+// are gone.  4096x4096 at 13 columns 8.8 -> 5.6 us, of which ~1.7 is the launch
 // and the rest two dependent step latencies a wave, not bandwidth (9.4 MB).
 //
 // Q5_K (176-byte blocks, 16-byte aligned like Q4_K) takes the Q4_K path with
@@ -225,9 +225,16 @@ constexpr int few_occupancy(int nst, int kh = 1) {
     return 163840 / (kh * nst * FewGeo<TYPE, NW, NCT, PACK>::STAGE + 16);
 }
 
+// waves per SIMD to keep registers for: those of the workgroups that the LDS holds
+template <int TYPE, int NW, int NCT, bool PACK>
+constexpr int few_waves(int nst, int kh) {
+    const int occ = few_occupancy<TYPE, NW, NCT, PACK>(nst, kh);
+    return nst == 1 ? occ * NW * kh / 4 : occ;
+}
+
 // KH K parts: the workgroup's waves are KH groups of NW, each over its share of
 // the workgroup's K-steps; the groups add their sums through LDS at the end,
-// group 0 first (deterministic).
+// as a fixed tree (deterministic).
 //   - NW = 4 waves, NST-stage rings (KH 1 or 2; the launcher makes the step count
 //     a multiple of KH, since the groups meet at every ring barrier): two waves
 //     with independent work share a SIMD.
@@ -235,7 +242,7 @@ constexpr int few_occupancy(int nst, int kh = 1) {
 //     and fills it again; no barrier until the sums meet, and the other waves of
 //     the CU cover the waits.
 template <int TYPE, int NST, int NW, int NCT, bool PACK, int KH, bool FUSED>
-__global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupancy<TYPE, NW, NCT, PACK>(NST, KH))) void mmq_few_kernel(
+__global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_waves<TYPE, NW, NCT, PACK>(NST, KH))) void mmq_few_kernel(
     const uint8_t *__restrict__ w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *__restrict__ yqs,
     const uint32_t *__restrict__ yds, int ncols, float *__restrict__ dst, int64_t dst_col_stride,
     float *__restrict__ partial, MmqGlu glu) {
@@ -306,11 +313,18 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupa
         }
     };
 
-    // The sums over K-steps.  A fused launch runs unsplit, so a lane adds up to 56
-    // steps in a row, which would round further from the f64 value than the 64-lane
-    // tree of the GEMV it replaces (4.4e-7 against 2.7e-7 of the result at K =
-    // 4096): it keeps the rounding errors of these additions (Knuth's two-sum) and
-    // adds them at the end (2.4e-7).  m is the min term's -dmin and P its sum.
+    // The sums over K-steps.  A fused or whole-K launch runs unsplit, so a lane adds
+    // up to 56 steps in a row, which would round further from the f64 value than the
+    // 64-lane tree of the GEMV or the split's shorter sums that it replaces: it keeps
+    // the rounding errors of these additions (Knuth's two-sum) and of the min product
+    // and adds them at the end, and sums a step's blocks in two halves.  Error over
+    // the result (2-norm), the replaced route / plain sums / these: fused Q4_K K =
+    // 4096 2.7e-7 / 4.4e-7 / 2.4e-7; whole K Q4_K 4096x14336 at 6 columns 1.8e-7 /
+    // 2.2e-7 / 1.1e-7, Q5_K 2048x8192 at 6 1.2e-7 / 1.9e-7 / 1.1e-7, Q4_0 4096x4096 at
+    // 8 7.4e-8 / 9.4e-8 / 6.7e-8.  It costs (us) Q4_K 4096x4096 at 13 7.4 -> 7.7, Q5_K
+    // 2048x8192 at 13 9.5 -> 10.5, Q4_0 4096x4096 at 8 7.7 -> 8.8 (from 10.0 on the
+    // GEMV).  m is the min term's -dmin and P its sum.
+    constexpr bool KEEP = FUSED || PRIVATE;
     v4f acc[NCT], lost[NCT];
 #pragma unroll
     for (int j = 0; j < NCT; ++j) acc[j] = lost[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -320,11 +334,15 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupa
         acc[j][v] = s;
     };
     auto add_step = [&](int j, int v, float d, float sum) {
-        if constexpr (FUSED) add_sum(j, v, d * sum);
+        if constexpr (KEEP) add_sum(j, v, d * sum);
         else acc[j][v] = fmaf(d, sum, acc[j][v]);
     };
     auto add_step_min = [&](int j, int v, float d, float sum, float m, float P) {
-        if constexpr (FUSED) add_sum(j, v, fmaf(d, sum, m * P));
+        if constexpr (KEEP) {
+            const float mP = m * P;
+            lost[j][v] += fmaf(m, P, -mP);
+            add_sum(j, v, fmaf(d, sum, mP));
+        }
         else acc[j][v] = fmaf(d, sum, fmaf(m, P, acc[j][v]));
     };
     // K-slot carriers: slot 0 and 2 of the scale MFMA live in lanes 0-15,
@@ -384,16 +402,14 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupa
                 const v4f SC = __builtin_amdgcn_mfma_f32_16x16x16f16(sa, scale_b(g, dh0[j], dh1[j]), zf, 0, 0, 0);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    if constexpr (FUSED) accb[j][v] = g == 0 ? (float)S[v] * SC[v] : fmaf((float)S[v], SC[v], accb[j][v]);
-                    else acc[j][v] = fmaf((float)S[v], SC[v], acc[j][v]);
+                    if constexpr (KEEP) {
+                        accb[j][v] = g % 4 == 0 ? (float)S[v] * SC[v] : fmaf((float)S[v], SC[v], accb[j][v]);
+                        if (g % 4 == 3) add_sum(j, v, accb[j][v]);
+                    } else {
+                        acc[j][v] = fmaf((float)S[v], SC[v], acc[j][v]);
+                    }
                 }
             }
-        }
-        if constexpr (FUSED) {
-#pragma unroll
-            for (int j = 0; j < NCT; ++j)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) add_sum(j, v, accb[j][v]);
         }
     };
 
@@ -464,7 +480,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupa
         uint4 dh0[NCT], dh1[NCT];
 #pragma unroll
         for (int j = 0; j < NCT; ++j) col_headers(st, j, bcol[j], dh0[j], dh1[j]);
-        v4f accb[NCT];
+        v4f accb[NCT], half[NCT];  // the step's sum, that of its first half
 #pragma unroll
         for (int g = 0; g < 8; ++g) {
             const uint2 q = *reinterpret_cast<const uint2 *>(blk + 8 + 16 * g + 8 * (kq & 1));
@@ -481,8 +497,11 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupa
                 const v4f zf = {0.0f, 0.0f, 0.0f, 0.0f};
                 const v4f SC = __builtin_amdgcn_mfma_f32_16x16x16f16(sa, scale_b(g, dh0[j], dh1[j]), zf, 0, 0, 0);
 #pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    accb[j][v] = g == 0 ? (float)S[v] * SC[v] : fmaf((float)S[v], SC[v], accb[j][v]);
+                for (int v = 0; v < 4; ++v) {
+                    if (KEEP && g == 4) half[j][v] = accb[j][v];
+                    accb[j][v] = g == 0 || (KEEP && g == 4) ? (float)S[v] * SC[v] : fmaf((float)S[v], SC[v], accb[j][v]);
+                    if (KEEP && g == 7) accb[j][v] += half[j][v];
+                }
             }
         }
         // d of the output rows (4*kq + v of this wave's 16)
@@ -579,7 +598,8 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupa
     // lane groups of its sub-block and zero in the other two, so every output
     // is a live (column, sub-block) dot, and the scale MFMA puts sc_{2c} * d8
     // in K slot 0 for columns 0-7 and sc_{2c+1} * d8 in slot 1 for columns
-    // 8-15.  The min term goes to columns 0-7 only, and the two halves of an
+    // 8-15.  Each half's min term covers its own sub-blocks (all eight in columns
+    // 0-7 left the halves two large sums that cancel), and the two halves of an
     // output column are added at the end.  Against one 16x16x32 MFMA per
     // sub-block with columns 8-15 idle, it halves the MFMAs and the
     // per-output convert + FMA of a step.
@@ -635,13 +655,14 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupa
 #pragma unroll
             for (int v = 0; v < 4; ++v) accb[v] = c == 0 ? (float)S[v] * SC[v] : fmaf((float)S[v], SC[v], accb[v]);
         }
-        // min term, columns 0-7 only: K slot 4*kq + t holds sub-block 4*kq + t for kq < 2
+        // min term: K slot 4*kq + t holds sub-block 4*kq + t for kq < 2, B the s8 of
+        // its column half's sub-blocks
         const uint32_t mb = ((kq & 1) ? mn_hi : mn_lo) & m_mn;
         const v4h am = __builtin_bit_cast(
             v4h, make_uint2(byte_f16(mb, 0) | (byte_f16(mb, 1) << 16), byte_f16(mb, 2) | (byte_f16(mb, 3) << 16)));
-        const uint32_t m_lo = phi ? 0u : 0xFFFFFFFFu;
-        const v4h bm = __builtin_bit_cast(v4h, make_uint2(__builtin_amdgcn_perm(dm.y, dm.x, 0x07060302u) & m_lo,
-                                                          __builtin_amdgcn_perm(dm.w, dm.z, 0x07060302u) & m_lo));
+        const uint32_t m_half = phi ? 0xFFFF0000u : 0x0000FFFFu;
+        const v4h bm = __builtin_bit_cast(v4h, make_uint2(__builtin_amdgcn_perm(dm.y, dm.x, 0x07060302u) & m_half,
+                                                          __builtin_amdgcn_perm(dm.w, dm.z, 0x07060302u) & m_half));
         const v4f zf = {0.0f, 0.0f, 0.0f, 0.0f};
         const v4f P = __builtin_amdgcn_mfma_f32_16x16x16f16(am, bm, zf, 0, 0, 0);
 #pragma unroll
@@ -738,14 +759,14 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupa
             }
         }
     }
-    if constexpr (FUSED) {
+    if constexpr (KEEP) {
 #pragma unroll
         for (int j = 0; j < NCT; ++j) acc[j] += lost[j];
     }
     if constexpr (KH > 1) {
         // every wave's stage reads (and transfers: the last wait was vmcnt(0))
         // are done; K parts 1.. hand their sums to part 0 through the stages'
-        // memory, which adds them in order
+        // memory, which adds them as a tree
         lds_barrier();
         v4f *part = reinterpret_cast<v4f *>(&rings[0][0][0]);
         if (kh > 0) {
@@ -755,9 +776,17 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_occupa
         lds_barrier();
         if (kh > 0) return;
 #pragma unroll
-        for (int k = 0; k < KH - 1; ++k)
+        for (int j = 0; j < NCT; ++j) {
+            v4f t[KH];
+            t[0] = acc[j];
 #pragma unroll
-            for (int j = 0; j < NCT; ++j) acc[j] += part[((k * NCT + j) * NW + wave) * 64 + lane];
+            for (int k = 1; k < KH; ++k) t[k] = part[(((k - 1) * NCT + j) * NW + wave) * 64 + lane];
+#pragma unroll
+            for (int h = 1; h < KH; h *= 2)
+#pragma unroll
+                for (int k = 0; k + h < KH; k += 2 * h) t[k] += t[k + h];
+            acc[j] = t[0];
+        }
     }
 
     // a lane's four rows of a column; fused, gate (v = 0, 1) and up (v = 2, 3) of two output rows
@@ -824,7 +853,8 @@ int mmq_few_split_k(int64_t K, int64_t nrows) {
 // columns' codes among 16 rows instead of 64, so the codes are most of what moves
 // into LDS and the 64-row tiles stay ahead on unsplit grids (>= 192 of them) and
 // where the weights stream long enough to hide the reduction.  Graph-timed,
-// kernel (+ reduction), 64-row tiles -> these, us at 13 columns unless given:
+// kernel (+ reduction), 64-row tiles -> these, us at 13 columns unless given (before
+// the kept rounding errors, which add 3-5 %, to Q5_K and Q4_0 10-15 %):
 //   Q4_K 4096x4096 at 4 / 13 / 32: 8.0 / 8.8 / 11.5 -> 5.5 / 5.3 / 7.0
 //   Q4_K 1024x4096 7.1 -> 4.7, 333x4096 9.7 -> 4.2, 256x256 3.2 -> 3.1
 //   Q4_K 4096x14336 at 4 / 13 / 24: 13.8 / 14.6 / 19.7 -> 11.8 / 13.0 / 18.0

@@ -1,7 +1,7 @@
 """The few-column GEMM whose 16-row workgroups hold all of K (at most 12224 rows and
 64 Mi weights, up to 32 columns; Q6_K 16), against the f64 Q8_1 formula at the edges
 of its tiles and K parts.  Each output sums exact integer dots with f32 scales: at
-most 8 terms a K step, 256 weights, then the steps and 8 parts in order, so the error
+most 8 terms a K step, 256 weights, then the steps and a tree of 8 parts, so the error
 is below (8 + K / 256 / 8 + 8) f32 half-ulps of the sum of |terms|, which is under 8
 times max |out| for these inputs: 24 * 6e-8 * 8 = 1.2e-5 at most; the shared gate of
 2e-6 of max |out| holds for the random signs."""
@@ -39,6 +39,25 @@ def test_few_whole_k(tname, nrows, K, ncols):
     np.testing.assert_array_equal(got, again)
     ideal = O.mul_mat_q8_1_f64(t, wq, nrows, K, G.quantize_q8_1(x_d, K).cpu().numpy(), ncols)
     assert max_err_scaled(got, ideal) < F64_TOL, max_err_scaled(got, ideal)
+
+
+@pytest.mark.parametrize("tname", list(TYPES))
+@pytest.mark.parametrize("ncols", [6, 13])
+def test_few_whole_k_precision(tname, ncols):
+    """Four steps a wave add no error that grows with the steps: below 2.75 f32 half-ulps
+    of the result's norm (a step's blocks, its min term and the result each round once;
+    plain sums measured 3.2 at 6 columns of Q4_K)."""
+    import ggml_hip as G
+    nrows, K = 2048, 8192
+    t = TYPES[tname]
+    wq = weights_q(t, nrows, K)
+    w_d = torch.from_numpy(np.array(wq)).cuda()
+    x_d = torch.from_numpy(np.array(acts(ncols, K))).cuda()
+    qs, ds = G.quantize_q8_1_planar(x_d)
+    got = G.mmq(tname, w_d, K, qs, ds).cpu().numpy().astype(np.float64)
+    ideal = O.mul_mat_q8_1_f64(t, wq, nrows, K, G.quantize_q8_1(x_d, K).cpu().numpy(), ncols)
+    rel = np.linalg.norm(got - ideal) / np.linalg.norm(ideal)
+    assert rel < 2.75 * 2.0 ** -24, rel * 2.0 ** 24
 
 
 @pytest.mark.parametrize("nrows", [12224, 12225])
