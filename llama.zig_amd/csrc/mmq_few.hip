@@ -345,10 +345,16 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_waves<
         }
         else acc[j][v] = fmaf(d, sum, fmaf(m, P, acc[j][v]));
     };
-    // K-slot carriers: slot 0 and 2 of the scale MFMA live in lanes 0-15,
-    // slots 0-7 of the min MFMA in lanes 0-31; the other lanes' A values are
-    // zero, so their (finite) B values add nothing.
+    // K-slot carriers: the scale MFMA's live slots are in lanes 0-15, the min
+    // MFMA's in lanes 0-31; the other slots add nothing because one side is zero and
+    // the other finite.  The columns' s8 must not stand beside a zero: a block whose
+    // 32 activations sum past 65504 (each 3000) has an infinite s8 with a finite d8,
+    // and zero times it is NaN.  So the scale MFMA's B holds d8 only; Q4_K and Q5_K
+    // above 8 columns keep the headers as stored, since their min term is infinite
+    // with such an s8 anyway (masked they took 2-4 % longer, Q5_K's whole-K form, whose
+    // registers then spill, 8-17 %).
     const uint32_t m_sc = kq == 0 ? 0xFFFFFFFFu : 0u;
+    const uint32_t m_d8 = m_sc & 0xFFFFu;
     const uint32_t m_mn = kq < 2 ? 0xFFFFFFFFu : 0u;
 
     // per column tile j: the lane's column 16j + li, its codes and its
@@ -359,15 +365,17 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_waves<
         dh0 = *reinterpret_cast<const uint4 *>(dcol);
         dh1 = *reinterpret_cast<const uint4 *>(dcol + 4);
     };
-    // the scale MFMA's B operand for block g: the headers of blocks 2h, 2h+1
-    // (h = g/2) as stored, d8 of block g in K slot 0 (g even) or 2 (g odd)
+    // the scale MFMA's B operand for block g: d8 of blocks g & ~1 and g | 1 in K slots
+    // 0 and 1 (one byte permute for the two; a mask for each took up to 5 % longer)
     auto scale_b = [&](int g, const uint4 &dh0, const uint4 &dh1) {
-        const uint4 &dh = g < 4 ? dh0 : dh1;
-        return __builtin_bit_cast(v4h, (g & 2) ? make_uint2(dh.z, dh.w) : make_uint2(dh.x, dh.y));
+        const uint4 dh = g < 4 ? dh0 : dh1;
+        const uint32_t lo = (g & 2) ? dh.z : dh.x, hi = (g & 2) ? dh.w : dh.y;
+        return __builtin_bit_cast(v4h, make_uint2(__builtin_amdgcn_perm(hi, lo, 0x05040100u), 0u));
     };
     // ... and its A operand: the row's f16 scale bits in the slot of block g
+    const uint32_t to_slot1 = kq == 0 ? 65536u : 0u;
     auto scale_a = [&](int g, uint32_t f16bits) {
-        return __builtin_bit_cast(v4h, (g & 1) ? make_uint2(0u, f16bits) : make_uint2(f16bits, 0u));
+        return __builtin_bit_cast(v4h, make_uint2((g & 1) ? __umul24(f16bits, to_slot1) : f16bits & m_sc, 0u));
     };
 
     auto compute_q8_0 = [&](const uint8_t *st) {
@@ -390,7 +398,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_waves<
             } else {
                 a = lds8_a2(blk + 2 + 8 * kq);
             }
-            const uint32_t dw = (uint32_t)*reinterpret_cast<const uint16_t *>(blk) & m_sc;
+            const uint32_t dw = (uint32_t)*reinterpret_cast<const uint16_t *>(blk);
             const v4h sa = scale_a(g, dw);
             const int c = 2 * g + (kq >> 1);
 #pragma unroll
@@ -437,8 +445,8 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_waves<
             const uint2 a_hi = kq < 2 ? make_uint2(0u, 0u) : make_uint2(v0, v1);
             // the row's int8 scales of sub-blocks 2g and 2g+1
             const uint32_t w2 = *reinterpret_cast<const uint16_t *>(blk + 192 + 2 * g);
-            const uint32_t sc0 = f16_bits((float)(int8_t)w2) & m_sc;
-            const uint32_t sc1 = f16_bits((float)(int8_t)(w2 >> 8)) & m_sc;
+            const uint32_t sc0 = f16_bits((float)(int8_t)w2);
+            const uint32_t sc1 = f16_bits((float)(int8_t)(w2 >> 8));
             const v4h sa0 = scale_a(g, sc0), sa1 = scale_a(g, sc1);
             const int c = 2 * g + (kq >> 1);
 #pragma unroll
@@ -487,7 +495,7 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_waves<
             const int sh = 4 * (kq >> 1);
             const uint2 a = make_uint2(iq4nl_levels((q.x >> sh) & 0x0F0F0F0Fu), iq4nl_levels((q.y >> sh) & 0x0F0F0F0Fu));
             const int ls = (int)(((hdr.y >> (4 * g)) & 0xFu) | (((hdr.x >> (16 + 2 * g)) & 3u) << 4)) - 32;
-            const v4h sa = scale_a(g, f16_bits((float)ls) & m_sc);
+            const v4h sa = scale_a(g, f16_bits((float)ls));
             const int c = 2 * g + (kq >> 1);
 #pragma unroll
             for (int j = 0; j < NCT; ++j) {
@@ -645,9 +653,9 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_waves<
             // A: (sc_{2c}, sc_{2c+1}) in K slots 0, 1 of lane group 0; B: d8 of block 2c + phi in slot phi
             const uint32_t scb = c < 2 ? sc_lo : sc_hi;
             const int sb = 16 * (c & 1);
-            const uint32_t sa2 = (byte_f16(scb >> sb, 0) | (byte_f16(scb >> sb, 1) << 16)) & m_sc;
+            const uint32_t sa2 = byte_f16(scb >> sb, 0) | (byte_f16(scb >> sb, 1) << 16);
             const uint4 &dh = c < 2 ? dh0 : dh1;
-            const uint32_t d8 = ((c & 1) ? (phi ? dh.w : dh.z) : (phi ? dh.y : dh.x)) & 0xFFFFu;
+            const uint32_t d8 = ((c & 1) ? (phi ? dh.w : dh.z) : (phi ? dh.y : dh.x)) & m_d8;
             const v4h sa = __builtin_bit_cast(v4h, make_uint2(sa2, 0u));
             const v4h sbv = __builtin_bit_cast(v4h, make_uint2(d8 << (16 * phi), 0u));
             const v4f zf = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -657,10 +665,10 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_waves<
         }
         // min term: K slot 4*kq + t holds sub-block 4*kq + t for kq < 2, B the s8 of
         // its column half's sub-blocks
-        const uint32_t mb = ((kq & 1) ? mn_hi : mn_lo) & m_mn;
+        const uint32_t mb = (kq & 1) ? mn_hi : mn_lo;
         const v4h am = __builtin_bit_cast(
             v4h, make_uint2(byte_f16(mb, 0) | (byte_f16(mb, 1) << 16), byte_f16(mb, 2) | (byte_f16(mb, 3) << 16)));
-        const uint32_t m_half = phi ? 0xFFFF0000u : 0x0000FFFFu;
+        const uint32_t m_half = (phi ? 0xFFFF0000u : 0x0000FFFFu) & m_mn;
         const v4h bm = __builtin_bit_cast(v4h, make_uint2(__builtin_amdgcn_perm(dm.y, dm.x, 0x07060302u) & m_half,
                                                           __builtin_amdgcn_perm(dm.w, dm.z, 0x07060302u) & m_half));
         const v4f zf = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -705,11 +713,11 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_waves<
             // A: the row's int8 scales of sub-blocks 2g, 2g+1 in K slots 0, 1 of
             // lane group 0; B: d8 of block g of column pj in slot phi
             const uint32_t w2 = *reinterpret_cast<const uint16_t *>(blk + 192 + 2 * g);
-            const uint32_t sa2 = (f16_bits((float)(int8_t)w2) | (f16_bits((float)(int8_t)(w2 >> 8)) << 16)) & m_sc;
+            const uint32_t sa2 = f16_bits((float)(int8_t)w2) | (f16_bits((float)(int8_t)(w2 >> 8)) << 16);
             const uint4 &dh = g < 4 ? dh0 : dh1;
             const uint32_t hw = (g & 2) ? ((g & 1) ? dh.w : dh.z) : ((g & 1) ? dh.y : dh.x);
             const v4h sa = __builtin_bit_cast(v4h, make_uint2(sa2, 0u));
-            const v4h sbv = __builtin_bit_cast(v4h, make_uint2((hw & 0xFFFFu) << (16 * phi), 0u));
+            const v4h sbv = __builtin_bit_cast(v4h, make_uint2((hw & m_d8) << (16 * phi), 0u));
             const v4f zf = {0.0f, 0.0f, 0.0f, 0.0f};
             const v4f SC = __builtin_amdgcn_mfma_f32_16x16x16f16(sa, sbv, zf, 0, 0, 0);
 #pragma unroll
