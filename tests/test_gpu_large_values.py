@@ -78,7 +78,7 @@ def test_glu_few_columns_overflowing_block_sums(tname, ncols):
 
 # up to 8 columns an infinite s of Q4_K / Q5_K times its mins is the formula's -inf
 @pytest.mark.parametrize("tname", list(MINS))
-@pytest.mark.parametrize("nrows,K,ncols", [(12300, 512, 4), (12300, 512, 8)])
+@pytest.mark.parametrize("nrows,K,ncols", [(12300, 512, 4), (12300, 512, 8), (6147, 1024, 8), (333, 4096, 5)])
 def test_few_columns_infinite_min_term(tname, nrows, K, ncols):
     import ggml_hip as G
     t = MINS[tname]
@@ -94,3 +94,63 @@ def test_few_columns_infinite_min_term(tname, nrows, K, ncols):
     assert np.isneginf(got[inf]).all()
     keep = ~inf.any(axis=1)
     assert max_err_scaled(got[keep], ideal[keep]) < F64_TOL
+
+
+def _infinite_block(tname, w, row, sb):
+    """256 weights of a row: an infinite f16 scale, positive codes and sub-block
+    scales, no min."""
+    nb = {"Q8_0": 34, "Q4_0": 18}.get(tname)
+    if nb:
+        blk = w[row, sb * 8 * nb:(sb * 8 + 1) * nb]
+        blk[:2] = (0x00, 0x7C)
+        blk[2:] = 0x7F if tname == "Q8_0" else 0xFF
+        return
+    size = O.BLOCK[O.TYPE_IDS[tname]][1]
+    blk = w[row, sb * size:(sb + 1) * size]
+    blk[:] = 0xFF  # largest codes
+    if tname == "Q6_K":
+        blk[192:208], blk[208:210] = 1, (0x00, 0x7C)
+    elif tname == "IQ4_XS":
+        blk[:2] = (0x00, 0x7C)
+    else:
+        blk[:4], blk[4:16] = (0x00, 0x7C, 0x00, 0x00), 0x11
+
+
+# whole-K (333 rows, 5 / 13 / 24 columns) and fused sums, which keep their rounding
+# errors, and the 64-row workgroups' plain ones
+@pytest.mark.parametrize("tname", list(NO_MINS) + list(MINS))
+@pytest.mark.parametrize("nrows,K,ncols", [(333, 4096, 5), (333, 4096, 13), (333, 4096, 24), (12300, 512, 5)])
+def test_few_columns_infinite_weight_scale(tname, nrows, K, ncols):
+    import ggml_hip as G
+    t = O.TYPE_IDS[tname]
+    w = _weights(t, nrows, K)
+    rows = [3, nrows - 1]
+    for i, r in enumerate(rows):
+        _infinite_block(tname, w, r, i)
+    x = np.abs(np.array(acts(ncols, K))) + 0.1
+    x[1::2] *= -1.0  # columns 1, 3, ..: -inf
+    x_d = torch.from_numpy(x).cuda()
+    pick = np.r_[0:100, nrows - 100:nrows]
+    ideal = _ideal(G, t, w[pick], x_d)
+    qs, ds = G.quantize_q8_1_planar(x_d)
+    got = G.mmq(tname, torch.from_numpy(w).cuda(), K, qs, ds).cpu().numpy()[:, pick]
+    bad = np.isin(pick, rows)
+    assert np.isposinf(ideal[0::2][:, bad]).all() and np.isneginf(ideal[1::2][:, bad]).all()
+    np.testing.assert_array_equal(got[:, bad], ideal[:, bad])
+    assert max_err_scaled(got[:, ~bad], ideal[:, ~bad]) < F64_TOL
+
+
+@pytest.mark.parametrize("ncols", [5, 13])
+def test_glu_few_columns_infinite_weight_scale(ncols):
+    """REGLU of an infinite gate and a positive finite up."""
+    import ggml_hip as G
+    t, nrows, K = O.TYPE_Q8_0, 6147, 2048
+    w, wg = _weights(t, nrows, K, 0), _weights(t, nrows, K, 1)
+    _infinite_block("Q8_0", wg, 3, 0)
+    x = np.abs(np.array(acts(ncols, K))) + 0.1
+    x_d = torch.from_numpy(x).cuda()
+    w_d, wg_d = torch.from_numpy(w).cuda(), torch.from_numpy(wg).cuda()
+    up = _ideal(G, t, w[:8], x_d)
+    got = G.mul_mat_glu("Q8_0", w_d, wg_d, x_d, "REGLU").cpu().numpy()
+    np.testing.assert_array_equal(got[:, 3], np.copysign(np.inf, up[:, 3]))
+    assert np.isfinite(np.delete(got, 3, axis=1)).all()
