@@ -4,6 +4,7 @@
 // ggml_cuda_mul_mat's choice between MMVQ and MMQ
 // (src/ggml/cuda/mulmat.zig:576-639; mmvq.zig:128-173; mmq.zig:865-917).
 #include "../../include/ggml_hip_qmm.h"
+#include "mmq_launch.h"
 #include "qmm_device.h"
 
 #include <atomic>
@@ -15,31 +16,6 @@ extern "C" int hip_qmm_mmq(int type, const void *w, int64_t K, int64_t nrows, in
                            const int8_t *y_qs, const void *y_ds, int64_t ncols, float *dst,
                            int64_t dst_col_stride, void *workspace, size_t workspace_size, void *stream);
 extern "C" size_t hip_qmm_mmq_workspace_size(int type, int64_t K, int64_t nrows, int64_t ncols);
-
-// mmq.hip: whether the few-column kernel takes this shape (given aligned operands)
-bool few_cols_type(int type, int64_t K, int64_t nrows, int64_t ncols);
-// mmq_few.hip: whether it takes these weight rows
-bool mmq_few_takes(int type, int64_t K, const void *w, int64_t row_stride);
-bool mmq_few_whole_k(int type, int64_t K, int64_t nrows, int64_t ncols);
-
-int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *yqs,
-                   const void *yds, int64_t ncols, float *dst, int64_t dst_col_stride, int split, float *partial,
-                   const MmqGlu &glu, hipStream_t s);
-// mmq.hip: its weight checks, and the sum of K-split partials
-int mmq_check_weights(int type, const void *w, int64_t K, int64_t row_stride);
-int mmq_add_partials(const float *partial, int split, int64_t nrows, int64_t ncols, float *dst, int64_t dst_col_stride,
-                     hipStream_t s);
-// mmq_f16.hip: the large-grid Q4_K / Q5_K / Q6_K GEMM on f16 matrix cores
-struct MmqF16Plan {
-    bool use, wide;
-    int split;
-};
-MmqF16Plan mmq_f16_plan(int type, int64_t K, int64_t nrows, int64_t ncols, bool glu);
-size_t mmq_f16_panel_bytes(int64_t K, int64_t ncols);
-int mmq_f16_quantize(const float *x, int64_t K, int64_t ncols, int64_t x_col_stride, void *panels, hipStream_t s);
-int mmq_f16_launch(int type, bool wide, const void *w, int64_t K, int64_t nrows, int64_t row_stride,
-                   const void *panels, int64_t ncols, float *dst, int64_t dst_col_stride, float *partial, int split,
-                   const MmqGlu &glu, hipStream_t s);
 
 // gemv.hip: 2-4 f32 columns (or twice the kernel's columns as two grid rows)
 // through the quantize-in-GEMV kernel, or hipErrorNotSupported for shapes it

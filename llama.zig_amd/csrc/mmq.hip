@@ -35,6 +35,7 @@
 
 #include "../../include/ggml_hip_qmm.h"
 #include "mmq_dma.h"
+#include "mmq_launch.h"
 #include "qmm_device.h"
 
 using namespace qmm;
@@ -57,13 +58,6 @@ int mmq_iq4xs_dma_launch(int bn, const void *w, int64_t K, int64_t nrows, int64_
 int mmq_q5k_dma_launch(int bn, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *yqs,
                        const void *yds, int64_t ncols, float *dst, int64_t dst_col_stride, dim3 grid, float *partial,
                        const qmm_dma::MmqGroups *grp, const MmqGlu &glu, hipStream_t s);
-// mmq_few.hip: the Q4_K / Q8_0 / Q6_K kernel for at most 32 columns
-int mmq_few_split_k(int64_t K, int64_t nrows);
-bool mmq_few_whole_k(int type, int64_t K, int64_t nrows, int64_t ncols);
-bool mmq_few_takes(int type, int64_t K, const void *w, int64_t row_stride);
-int mmq_few_launch(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *yqs,
-                   const void *yds, int64_t ncols, float *dst, int64_t dst_col_stride, int split, float *partial,
-                   const MmqGlu &glu, hipStream_t s);
 
 namespace {
 

@@ -36,6 +36,7 @@
 
 #include "../../include/ggml_hip_qmm.h"
 #include "mmq_dma.h"
+#include "mmq_launch.h"
 #include "qmm_device.h"
 
 using namespace qmm;
@@ -483,11 +484,6 @@ int launch_type(bool wide, const void *w, int64_t K, int64_t nrows, int64_t row_
 // (4096x4096 at 200 / 512: 28 / 41 against 37 / 45; 14336x4096 at 128 / 256: 37 /
 // 57 against 41 / 61), whose nibbles they unpack for a fraction of what the
 // decoding here costs on few column tiles.
-struct MmqF16Plan {
-    bool use, wide;
-    int split;
-};
-
 MmqF16Plan mmq_f16_plan(int type, int64_t K, int64_t nrows, int64_t ncols, bool glu) {
     MmqF16Plan best{false, false, 1};
     if ((type != TYPE_Q4_K && type != TYPE_Q5_K && type != TYPE_Q6_K) || K <= 0 || K % QK_K != 0 || K > (1 << 30) ||

@@ -71,6 +71,7 @@
 // (l % 16) of B over the K-slice [(l / 16) * K/4, +K/4); the result value i of
 // lane l is row 4*(l/16) + i, column l % 16.
 #include "../../include/ggml_hip_qmm.h"
+#include "mmq_launch.h"
 #include "qmm_device.h"
 
 using namespace qmm;
