@@ -338,6 +338,11 @@ int hip_qmm_mul_mat_noalloc(int type, const void *w, int64_t K, int64_t nrows, i
  * over several workgroups (the reference's stream-k fixup, mmq.zig:359-407)
  * and the partials, kept in `workspace`, are summed in a fixed order; with
  * no or too small a workspace the GEMM runs unsplit.
+ * Above 32 columns (and in the grouped and gate/up forms below) the tiles of
+ * Q8_0, Q4_0 and IQ4_XS multiply a header's s, which those types do not use,
+ * by zero: an infinite s (a block of activations that sums past 65504) gives
+ * NaN there.  Clear the headers' upper halves for them, as hip_qmm_mul_mat and
+ * its relatives do in their own copy of x.
  */
 int hip_qmm_mmq(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride, const int8_t *y_qs,
                 const void *y_ds, int64_t ncols, float *dst, int64_t dst_col_stride, void *workspace,

@@ -269,7 +269,8 @@ extern "C" int hip_qmm_mul_mat(int type, const void *w, int64_t K, int64_t nrows
     const int64_t Kp = pad_k(K);
     int8_t *qs = (int8_t *)workspace;
     void *ds = (uint8_t *)workspace + ncols * Kp;
-    if (int e = hip_qmm_quantize_q8_1_planar(x, K, ncols, x_col_stride, qs, ds, stream)) return e;
+    if (int e = qmm_quantize_planar(x, K, ncols, x_col_stride, qs, ds, q8_1_header_mask(type), (hipStream_t)stream))
+        return e;
     if (ncols <= 8 && !use_mmq_rows(type, K, nrows, ncols, w, row_stride))
         return hip_qmm_mul_mat_vec(type, w, K, nrows, row_stride, qs, ds, ncols, dst, dst_col_stride, stream);
     if (K % 256 == 0) {
@@ -329,7 +330,8 @@ extern "C" int hip_qmm_mul_mat_glu(int type, const void *w, const void *w_gate, 
         const int64_t Kp = pad_k(K);
         int8_t *qs = (int8_t *)workspace;
         void *ds = (uint8_t *)workspace + ncols * Kp;
-        if (int e = hip_qmm_quantize_q8_1_planar(x, K, ncols, x_col_stride, qs, ds, stream)) return e;
+        if (int e = qmm_quantize_planar(x, K, ncols, x_col_stride, qs, ds, q8_1_header_mask(type), (hipStream_t)stream))
+            return e;
         return hip_qmm_mmq_glu(type, w, w_gate, K, nrows, row_stride, qs, ds, ncols, glu_op, glu_alpha, glu_limit,
                                dst, dst_col_stride, stream);
     }
@@ -339,7 +341,8 @@ extern "C" int hip_qmm_mul_mat_glu(int type, const void *w, const void *w_gate, 
         const int64_t Kp = pad_k(K);
         int8_t *qs = (int8_t *)workspace;
         void *ds = (uint8_t *)workspace + ncols * Kp;
-        if (int e = hip_qmm_quantize_q8_1_planar(x, K, ncols, x_col_stride, qs, ds, stream)) return e;
+        if (int e = qmm_quantize_planar(x, K, ncols, x_col_stride, qs, ds, q8_1_header_mask(type), (hipStream_t)stream))
+            return e;
         const MmqGlu glu{(const uint8_t *)w_gate, glu_op, glu_alpha, glu_limit};
         return mmq_few_launch(type, w, K, nrows, row_stride, qs, ds, ncols, dst, dst_col_stride, 1, nullptr, glu,
                               (hipStream_t)stream);

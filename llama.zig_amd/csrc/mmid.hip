@@ -12,6 +12,7 @@
 // Ids outside [-1, n_as) are treated as -1 (zero row) rather than read out
 // of bounds.
 #include "../../include/ggml_hip_qmm.h"
+#include "mmq_launch.h"
 #include "qmm_device.h"
 
 using namespace qmm;
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(PREP_THREADS) void mmid_prepare(
     int32_t *__restrict__ tiles, int32_t *__restrict__ n_tiles,
     float *__restrict__ dst, int64_t dst_row_stride, int64_t nrows, const float *__restrict__ x, int64_t K,
     int64_t x_row_stride, int64_t Kp, int nq_per_row, int rows_per_wg, int64_t nrows_x, int8_t *__restrict__ qs,
-    uint32_t *__restrict__ ds) {
+    uint32_t *__restrict__ ds, uint32_t keep) {
     const int tid = threadIdx.x;
     if ((int)blockIdx.x >= n_group) {
         // quantize: workgroup (row, K slice of QUANT_VALS values), or for rows
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(PREP_THREADS) void mmid_prepare(
         }
         const Q8Quad r = q8_1_quantize_quad(v);
         *reinterpret_cast<uint2 *>(qs + c * Kp + k) = make_uint2(r.lo, r.hi);
-        if ((tid & 3) == 0) ds[c * (Kp / QK8) + k / QK8] = r.ds;
+        if ((tid & 3) == 0) ds[c * (Kp / QK8) + k / QK8] = r.ds & keep;
         return;
     }
 
@@ -413,6 +414,7 @@ int mul_mat_id(int type, const void *w, const void *w_gate, int64_t K, int64_t n
     hipStream_t s = (hipStream_t)stream;
 
     const int n_group = n_as < 256 ? (int)n_as : 256;
+    const uint32_t keep = q8_1_header_mask(type);
     if ((uintptr_t)x % 16 == 0 && x_row_stride % 4 == 0 && K % QK8 == 0) {
         // one launch: grouping and quantization
         const int nq_per_row = (int)((L.Kp + QUANT_VALS - 1) / QUANT_VALS);
@@ -424,12 +426,13 @@ int mul_mat_id(int type, const void *w, const void *w_gate, int64_t K, int64_t n
         hipLaunchKernelGGL(mmid_prepare, dim3((unsigned)nwg), dim3(PREP_THREADS), 0, s, ids, ids_stride, n_tokens,
                            n_ids, (int)n_as, ne11, bn, n_group, col_src, col_dst, tiles, ntiles, dst,
                            dst_row_stride, nrows, x, K, x_row_stride, L.Kp, nq_per_row, rows_per_wg, L.nrows_x, qs,
-                           (uint32_t *)ds);
+                           (uint32_t *)ds, keep);
     } else {
-        if (int e = hip_qmm_quantize_q8_1_planar(x, K, L.nrows_x, x_row_stride, qs, ds, stream)) return e;
+        if (int e = qmm_quantize_planar(x, K, L.nrows_x, x_row_stride, qs, ds, keep, s)) return e;
         hipLaunchKernelGGL(mmid_prepare, dim3((unsigned)n_group), dim3(PREP_THREADS), 0, s, ids, ids_stride, n_tokens,
                            n_ids, (int)n_as, ne11, bn, n_group, col_src, col_dst, tiles, ntiles, dst,
-                           dst_row_stride, nrows, x, K, x_row_stride, L.Kp, 1, 1, L.nrows_x, qs, (uint32_t *)ds);
+                           dst_row_stride, nrows, x, K, x_row_stride, L.Kp, 1, 1, L.nrows_x, qs, (uint32_t *)ds,
+                           keep);
     }
     if (int e = (int)hipGetLastError()) return e;
     if (w_gate)

@@ -9,6 +9,11 @@
 
 #include "qmm_device.h"
 
+// quantize_q8_1.hip: hip_qmm_quantize_q8_1_planar with the header bits of `keep` only
+// (q8_1_header_mask of the weights' type for an op's own copy)
+int qmm_quantize_planar(const float *x, int64_t K, int64_t ncols, int64_t x_col_stride, int8_t *qs, void *ds,
+                        uint32_t keep, hipStream_t s);
+
 // mmq.hip: whether the few-column kernel takes this shape (given aligned operands),
 // the weight checks of its dispatch, and the sum of K-split partials
 bool few_cols_type(int type, int64_t K, int64_t nrows, int64_t ncols);

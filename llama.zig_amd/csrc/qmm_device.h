@@ -170,6 +170,13 @@ __device__ __forceinline__ float quad_x2(float v) {
 __device__ __forceinline__ int quad_x1(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false); }
 __device__ __forceinline__ int quad_x2(int v) { return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false); }
 
+// The part of a Q8_1 header that weights of this type read: d, and s only for the
+// types with mins.  An op's own Q8_1 copy keeps no more: s is infinite where a block's
+// activations sum past 65504, and the MMQ tiles pair it with a zero (NaN).
+__host__ __device__ constexpr uint32_t q8_1_header_mask(int type) {
+    return type == TYPE_Q4_K || type == TYPE_Q5_K ? 0xFFFFFFFFu : 0xFFFFu;
+}
+
 // One Q8_1 block held by the 4 lanes of a quad, 8 consecutive values per lane
 // (quantize_row_q8_1_ref, src/ggml/quants/legacy.zig:451-484): amax and the
 // code sum take two DPP exchanges each; the max and the integer sum do not

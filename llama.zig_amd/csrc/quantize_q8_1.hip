@@ -9,6 +9,7 @@
 // One 32-lane half-wave per Q8_1 block: lane i owns element i of the block;
 // amax and sum(q) are butterfly reductions inside the half-wave.
 #include "../../include/ggml_hip_qmm.h"
+#include "mmq_launch.h"
 #include "qmm_device.h"
 
 using namespace qmm;
@@ -51,17 +52,18 @@ __global__ __launch_bounds__(256) void quantize_q8_1_aos(const float *__restrict
     if ((i0 & 31) == 0) *reinterpret_cast<uint32_t *>(blk) = q8_1_pack_ds(v.d, v.sum);
 }
 
-// Planar output: qs[c*Kp + k], ds[c*Kp/32 + k/32].
+// Planar output: qs[c*Kp + k], ds[c*Kp/32 + k/32] (its bits of `keep`).
 __global__ __launch_bounds__(256) void quantize_q8_1_planar(const float *__restrict__ x, int64_t K,
                                                             int64_t x_col_stride, int64_t Kp,
-                                                            int8_t *__restrict__ qs, uint32_t *__restrict__ ds) {
+                                                            int8_t *__restrict__ qs, uint32_t *__restrict__ ds,
+                                                            uint32_t keep) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t c = blockIdx.y;
     if (k >= Kp) return;
     const float xv = k < K ? x[c * x_col_stride + k] : 0.0f;
     const Q8_1Val v = quantize_lane32(xv);
     qs[c * Kp + k] = v.q;
-    if ((k & 31) == 0) ds[c * (Kp / QK8) + k / QK8] = q8_1_pack_ds(v.d, v.sum);
+    if ((k & 31) == 0) ds[c * (Kp / QK8) + k / QK8] = q8_1_pack_ds(v.d, v.sum) & keep;
 }
 
 // Planar output, 8 consecutive values per lane: a 32-block is the 4 lanes of
@@ -71,7 +73,8 @@ __global__ __launch_bounds__(256) void quantize_q8_1_planar(const float *__restr
 // kernel's.  Needs x 16-byte aligned and x_col_stride a multiple of 4.
 __global__ __launch_bounds__(256) void quantize_q8_1_planar8(const float *__restrict__ x, int64_t K,
                                                              int64_t x_col_stride, int64_t Kp,
-                                                             int8_t *__restrict__ qs, uint32_t *__restrict__ ds) {
+                                                             int8_t *__restrict__ qs, uint32_t *__restrict__ ds,
+                                                             uint32_t keep) {
     const int64_t k = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
     const int64_t c = blockIdx.y;
     // whole quads stay active: Kp is a multiple of 512, so k < Kp for all 4 lanes or none
@@ -88,7 +91,7 @@ __global__ __launch_bounds__(256) void quantize_q8_1_planar8(const float *__rest
     }
     const Q8Quad r = q8_1_quantize_quad(v);
     *reinterpret_cast<uint2 *>(qs + c * Kp + k) = make_uint2(r.lo, r.hi);
-    if ((threadIdx.x & 3) == 0) ds[c * (Kp / QK8) + k / QK8] = r.ds;
+    if ((threadIdx.x & 3) == 0) ds[c * (Kp / QK8) + k / QK8] = r.ds & keep;
 }
 
 }  // namespace
@@ -106,20 +109,25 @@ extern "C" int hip_qmm_quantize_q8_1(const float *x, void *y_q8_1, int64_t ne00,
     return (int)hipGetLastError();
 }
 
-extern "C" int hip_qmm_quantize_q8_1_planar(const float *x, int64_t K, int64_t ncols, int64_t x_col_stride,
-                                            int8_t *qs, void *ds, void *stream) {
+int qmm_quantize_planar(const float *x, int64_t K, int64_t ncols, int64_t x_col_stride, int8_t *qs, void *ds,
+                        uint32_t keep, hipStream_t s) {
     if (!x || !qs || !ds || K <= 0 || K % QK8 != 0 || ncols < 0 || ncols > 65535 || x_col_stride < K)
         return (int)hipErrorInvalidValue;
     if (ncols == 0) return 0;
     const int64_t Kp = pad_k(K);
     if ((uintptr_t)x % 16 == 0 && x_col_stride % 4 == 0 && (uintptr_t)qs % 8 == 0) {
         const dim3 grid((unsigned)((Kp / 8 + 255) / 256), (unsigned)ncols);
-        hipLaunchKernelGGL(quantize_q8_1_planar8, grid, dim3(256), 0, (hipStream_t)stream, x, K, x_col_stride, Kp, qs,
-                           (uint32_t *)ds);
+        hipLaunchKernelGGL(quantize_q8_1_planar8, grid, dim3(256), 0, s, x, K, x_col_stride, Kp, qs, (uint32_t *)ds,
+                           keep);
     } else {
         const dim3 grid((unsigned)((Kp + 255) / 256), (unsigned)ncols);
-        hipLaunchKernelGGL(quantize_q8_1_planar, grid, dim3(256), 0, (hipStream_t)stream, x, K, x_col_stride, Kp, qs,
-                           (uint32_t *)ds);
+        hipLaunchKernelGGL(quantize_q8_1_planar, grid, dim3(256), 0, s, x, K, x_col_stride, Kp, qs, (uint32_t *)ds,
+                           keep);
     }
     return (int)hipGetLastError();
+}
+
+extern "C" int hip_qmm_quantize_q8_1_planar(const float *x, int64_t K, int64_t ncols, int64_t x_col_stride,
+                                            int8_t *qs, void *ds, void *stream) {
+    return qmm_quantize_planar(x, K, ncols, x_col_stride, qs, ds, 0xFFFFFFFFu, (hipStream_t)stream);
 }

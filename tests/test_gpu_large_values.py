@@ -76,6 +76,46 @@ def test_glu_few_columns_overflowing_block_sums(tname, ncols):
     assert np.abs(got.cpu().numpy()[:, rows] - np.maximum(gate, 0.0) * up).max() < bound
 
 
+# the MMQ tiles: an op's own Q8_1 copy leaves s out for these types
+@pytest.mark.parametrize("tname", list(NO_MINS))
+@pytest.mark.parametrize("nrows,K,ncols", [(333, 2048, 40), (1030, 4096, 200)])
+def test_tiles_overflowing_block_sums(tname, nrows, K, ncols):
+    import ggml_hip as G
+    t = NO_MINS[tname]
+    w = _weights(t, nrows, K)
+    x = _overflowing(ncols, K)
+    w_d, x_d = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()
+    xu = torch.empty(ncols * K + 1, device="cuda")[1:].view(ncols, K)  # not 16-byte aligned: the plain quantizer
+    xu.copy_(x_d)
+    rows = np.r_[0:100, nrows - 100:nrows]
+    ideal = _ideal(G, t, w[rows], x_d)
+    for got in (G.mul_mat(tname, w_d, x_d), G.mul_mat(tname, w_d, xu)):
+        assert torch.isfinite(got).all()
+        assert max_err_scaled(got.cpu().numpy()[:, rows], ideal) < F64_TOL
+    gated = G.mul_mat_glu(tname, w_d, torch.from_numpy(_weights(t, nrows, K, 1)).cuda(), x_d, "REGLU")
+    assert torch.isfinite(gated).all()
+
+
+@pytest.mark.parametrize("tname", list(NO_MINS))
+def test_mul_mat_id_overflowing_block_sums(tname):
+    import ggml_hip as G
+    from cases import mul_mat_id_f64, route_top_k
+    t, n_as, nrows, K, n_tokens = NO_MINS[tname], 4, 96, 1024, 40
+    w = np.stack([weights_q(t, nrows, K, i) for i in range(n_as)])
+    x = _overflowing(n_tokens, K)
+    ids = route_top_k(n_tokens, n_as, 2)[0]
+    w_d, ids_d = torch.from_numpy(w).cuda(), torch.from_numpy(ids).cuda()
+    xu = torch.empty(n_tokens * K + 1, device="cuda")[1:].view(n_tokens, 1, K)  # not 16-byte aligned
+    xu.copy_(torch.from_numpy(x).view(n_tokens, 1, K))
+    x_d = xu.clone()
+    ideal = mul_mat_id_f64(t, w, nrows, K, G.quantize_q8_1(x_d.view(n_tokens, K), K).cpu().numpy(), 1, ids)
+    for v in (x_d, xu):
+        got = G.mul_mat_id(tname, w_d, v, ids_d)
+        assert torch.isfinite(got).all()
+        assert max_err_scaled(got.cpu().numpy(), ideal) < F64_TOL
+    assert torch.isfinite(G.mul_mat_id_glu(tname, w_d, w_d, x_d, ids_d, "REGLU")).all()
+
+
 # up to 8 columns an infinite s of Q4_K / Q5_K times its mins is the formula's -inf
 @pytest.mark.parametrize("tname", list(MINS))
 @pytest.mark.parametrize("nrows,K,ncols", [(12300, 512, 4), (12300, 512, 8), (6147, 1024, 8), (333, 4096, 5)])
