@@ -79,8 +79,9 @@ size_t hip_qmm_mul_mat_workspace_size(int type, int64_t K, int64_t nrows, int64_
  * shape: at least hip_qmm_mul_mat_workspace_size, more where the f16 GEMM
  * (mmq_f16.hip, large grids of Q4_K, Q5_K and Q6_K above 32 columns) takes the
  * columns as panels.  With less, down to hip_qmm_mul_mat_workspace_size, the
- * int8 MMQ runs.  hip_qmm_mul_mat_glu_workspace_preferred: the same for
- * hip_qmm_mul_mat_glu. */
+ * int8 MMQ runs: its results are the same bits for Q4_K and Q5_K where neither
+ * splits K, and differ in fp32 rounding otherwise.
+ * hip_qmm_mul_mat_glu_workspace_preferred: the same for hip_qmm_mul_mat_glu. */
 size_t hip_qmm_mul_mat_workspace_preferred(int type, int64_t K, int64_t nrows, int64_t ncols);
 size_t hip_qmm_mul_mat_glu_workspace_preferred(int type, int64_t K, int64_t nrows, int64_t ncols);
 
@@ -307,20 +308,24 @@ int hip_qmm_mul_mat(int type, const void *w, int64_t K, int64_t nrows, int64_t r
                     const float *x, int64_t ncols, int64_t x_col_stride, float *dst,
                     int64_t dst_col_stride, void *workspace, size_t workspace_size, void *stream);
 
-/* Scratch bytes behind hip_qmm_mul_mat_noalloc, per device (32 MiB). */
+/* Most bytes of hip_qmm_mul_mat_workspace_size that hip_qmm_mul_mat_noalloc
+ * accepts (32 MiB), and the scratch behind it per device (128 MiB: what
+ * hip_qmm_mul_mat_workspace_preferred asks for such a shape is at most 114). */
 #define HIP_QMM_NOALLOC_SCRATCH_BYTES (32u << 20)
+#define HIP_QMM_NOALLOC_ARRAY_BYTES (128u << 20)
 
 /*
  * hip_qmm_mul_mat without the workspace arguments: the same dispatch, the
- * same kernels and the same results, with its scratch (the Q8_1 copy of x and
- * any split-K partials) in a fixed device array of
- * HIP_QMM_NOALLOC_SCRATCH_BYTES that each device holds for the life of the
+ * same kernels and the same results as with
+ * hip_qmm_mul_mat_workspace_preferred bytes, with its scratch (the copy of x
+ * that the kernel reads and any split-K partials) in a fixed device array of
+ * HIP_QMM_NOALLOC_ARRAY_BYTES that each device holds for the life of the
  * process.  It calls no hipMalloc / hipFree or anything that allocates; the
  * array's address is looked up once per device on the first call with that
  * device current.  Uses the current device's array: `stream` must belong to
  * the current device.  Shapes whose workspace
- * (hip_qmm_mul_mat_workspace_size) exceeds the array are rejected with
- * hipErrorInvalidValue before any launch.  All calls on one device share the
+ * (hip_qmm_mul_mat_workspace_size) exceeds HIP_QMM_NOALLOC_SCRATCH_BYTES are
+ * rejected with hipErrorInvalidValue before any launch.  All calls on one device share the
  * array, so calls that may overlap on one GPU (different streams, threads)
  * race; calls in one stream's order do not.
  * No counterpart in the reference: an entry point for callers that cannot

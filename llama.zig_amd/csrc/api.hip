@@ -371,8 +371,15 @@ extern "C" int hip_qmm_mul_mat_glu(int type, const void *w, const void *w_gate, 
 // Every call on one device shares its array: calls that overlap on one GPU
 // race, and a call leaves its scratch contents behind (nothing in the op
 // reads scratch before writing it, so no clearing is needed).
+//
+// The array holds hip_qmm_mul_mat_workspace_preferred of every shape that is
+// accepted, so the kernel, and with it the result, is that of a call with that
+// workspace.  A required size of 32 MiB bounds ncols * K * 9/8, so the f16 route's
+// panels, 288 K bytes for each 128 columns begun, take at most 64 MiB + 288 K, 82
+// MiB with its K <= 65536, and its K split's partials, of at most 256 tiles of 256 x
+// 128 f32, at most 32 MiB.
 
-static __device__ __align__(256) uint8_t scratch[HIP_QMM_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) uint8_t scratch[HIP_QMM_NOALLOC_ARRAY_BYTES];
 
 namespace {
 constexpr int MAX_DEVICES = 64;
@@ -407,5 +414,5 @@ extern "C" int hip_qmm_mul_mat_noalloc(int type, const void *w, int64_t K, int64
     void *ws = nullptr;
     if (int e = current_device_scratch(&ws)) return e;
     return hip_qmm_mul_mat(type, w, K, nrows, row_stride, x, ncols, x_col_stride, dst, dst_col_stride, ws,
-                           (size_t)HIP_QMM_NOALLOC_SCRATCH_BYTES, stream);
+                           (size_t)HIP_QMM_NOALLOC_ARRAY_BYTES, stream);
 }

@@ -51,6 +51,8 @@ constexpr int PANEL_D = 16384;       // d8 * 2^24: [sub-block / 4][column][sub-b
 constexpr int PANEL_S = 17408;       // s8: [column][sub-block] f16
 constexpr int PANEL_UNIT = 4;        // panels per super-block are a multiple of this (the widest tile)
 
+constexpr int F16_MAX_K = 65536;  // keeps the panels of a call without a workspace argument within its array (api.hip)
+
 constexpr int F16_CUS = 256;   // 256 x 128 tiles resident at once, one per CU
 constexpr int F16_REST = 128;  // a last round of at most this many tiles runs as quarter tiles
 
@@ -486,7 +488,7 @@ int launch_type(bool wide, const void *w, int64_t K, int64_t nrows, int64_t row_
 // decoding here costs on few column tiles.
 MmqF16Plan mmq_f16_plan(int type, int64_t K, int64_t nrows, int64_t ncols, bool glu) {
     MmqF16Plan best{false, false, 1};
-    if ((type != TYPE_Q4_K && type != TYPE_Q5_K && type != TYPE_Q6_K) || K <= 0 || K % QK_K != 0 || K > (1 << 30) ||
+    if ((type != TYPE_Q4_K && type != TYPE_Q5_K && type != TYPE_Q6_K) || K <= 0 || K % QK_K != 0 || K > F16_MAX_K ||
         nrows <= 0 || nrows > 0x7FFFFFFF || ncols <= 32 || ncols > 65535)
         return best;
     const bool q6 = type == TYPE_Q6_K, q5 = type == TYPE_Q5_K;
