@@ -274,9 +274,11 @@ extern "C" int hip_qmm_mul_mat(int type, const void *w, int64_t K, int64_t nrows
     if (ncols <= 8 && !use_mmq_rows(type, K, nrows, ncols, w, row_stride))
         return hip_qmm_mul_mat_vec(type, w, K, nrows, row_stride, qs, ds, ncols, dst, dst_col_stride, stream);
     if (K % 256 == 0) {
+        // few-column calls without partials may end before the aligned offset
         const size_t off = align256(q8_1_bytes(K, ncols));
-        return hip_qmm_mmq(type, w, K, nrows, row_stride, qs, ds, ncols, dst, dst_col_stride, (uint8_t *)workspace + off,
-                           workspace_size - off, stream);
+        const bool rest = workspace_size > off;
+        return hip_qmm_mmq(type, w, K, nrows, row_stride, qs, ds, ncols, dst, dst_col_stride,
+                           rest ? (uint8_t *)workspace + off : nullptr, rest ? workspace_size - off : 0, stream);
     }
     // Q8_0 / Q4_0 rows whose length is not a multiple of 256 (the MMQ K-step):
     // GEMV over column groups of 8.
