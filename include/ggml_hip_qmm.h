@@ -89,16 +89,33 @@ size_t hip_qmm_mul_mat_glu_workspace_preferred(int type, int64_t K, int64_t nrow
  * rather than the GEMV for this shape on 16-byte-aligned rows, else 0 (the
  * shape rules that hip_qmm_mul_mat_workspace_size applies; 3-8 columns of
  * 2048-12224 rows also run the few-column GEMM's form that needs no workspace
- * beyond the Q8_1 planes where that is faster, with 0 here).  No counterpart
- * in the reference: a query for measurement and tests that time or check the
- * kernel the op takes. */
+ * beyond the Q8_1 planes where that is faster, with 0 here: hip_qmm_kernel
+ * names the kernel).  No counterpart in the reference. */
 int hip_qmm_mul_mat_uses_mmq(int type, int64_t K, int64_t nrows, int64_t ncols);
+
+/* The kernel that an op runs for a shape, on operands aligned to 16 bytes and with
+ * the preferred workspace; -1 where the op takes no such shape.  op:
+ * HIP_QMM_OP_MUL_MAT, _MUL_MAT_GLU (hip_qmm_mul_mat_glu) or _MMQ (hip_qmm_mmq).
+ * _FEW is the few-column GEMM in 64-row workgroups, _FEW_WHOLE_K in 16-row ones
+ * that hold all of K, _TILE the int8 MMQ tiles, _F16 the f16 GEMM; _GEMV stands
+ * for every GEMV form, _UNFUSED for two products and the GLU kernel.  No
+ * counterpart in the reference: for measurement and tests. */
+enum { HIP_QMM_OP_MUL_MAT = 0, HIP_QMM_OP_MUL_MAT_GLU = 1, HIP_QMM_OP_MMQ = 2 };
+enum {
+    HIP_QMM_KERNEL_GEMV = 0,
+    HIP_QMM_KERNEL_FEW = 1,
+    HIP_QMM_KERNEL_FEW_WHOLE_K = 2,
+    HIP_QMM_KERNEL_TILE = 3,
+    HIP_QMM_KERNEL_F16 = 4,
+    HIP_QMM_KERNEL_UNFUSED = 5
+};
+int hip_qmm_kernel(int op, int type, int64_t K, int64_t nrows, int64_t ncols);
 
 /* 1 if hip_qmm_mul_mat runs these 2-8 f32 columns as rows of the one-column
  * fused kernel's grid (each column quantized in the kernel and equal bit for
  * bit to hip_qmm_mul_mat_vec_f32 on it; 16-byte-aligned x with a column
  * stride of a multiple of 4 floats), else 0.  No counterpart in the reference:
- * a query for measurement and tests, like hip_qmm_mul_mat_uses_mmq. */
+ * a query for measurement and tests, like hip_qmm_kernel. */
 int hip_qmm_mul_mat_per_column(int type, int64_t K, int64_t nrows, int64_t ncols);
 
 /*
@@ -408,7 +425,8 @@ size_t hip_qmm_mul_mat_glu_workspace_size(int type, int64_t K, int64_t nrows, in
 
 /* 1 if hip_qmm_mul_mat_glu runs a fused MMQ for this shape (the products
  * would each run the MMQ tile kernel, or, above 8 columns, the few-column GEMM
- * takes both weights in one launch), else 0: the reference's
+ * takes both weights in one launch; at 2-8 columns, where it does too on the
+ * shapes that hip_qmm_kernel names, 0), else 0: the reference's
  * shouldFuseMulMatQ (src/ggml/cuda/mulmat.zig:548-571) for this backend. */
 int hip_qmm_mul_mat_glu_fused(int type, int64_t K, int64_t nrows, int64_t ncols);
 

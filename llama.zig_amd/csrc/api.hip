@@ -237,6 +237,26 @@ extern "C" int hip_qmm_mul_mat_uses_mmq(int type, int64_t K, int64_t nrows, int6
     return K > 0 && nrows > 0 && ncols > 1 && use_mmq(type, K, nrows, ncols) ? 1 : 0;
 }
 
+extern "C" int hip_qmm_kernel(int op, int type, int64_t K, int64_t nrows, int64_t ncols) {
+    const bool legacy = type == TYPE_Q8_0 || type == TYPE_Q4_0;
+    const bool known = legacy || type == TYPE_Q4_K || type == TYPE_Q5_K || type == TYPE_Q6_K || type == TYPE_IQ4_XS;
+    if (!known || K <= 0 || nrows <= 0 || ncols <= 0 || K % (legacy ? QK8 : QK_K)) return -1;
+    if (op == HIP_QMM_OP_MMQ) return K % QK_K ? -1 : mmq_kernel_of(type, K, nrows, ncols);
+    if (op == HIP_QMM_OP_MUL_MAT) {
+        if (ncols == 1 || K % QK_K || !(use_mmq(type, K, nrows, ncols) || few_whole_wins(type, K, nrows, ncols)))
+            return HIP_QMM_KERNEL_GEMV;
+        return ncols > 8 && mmq_f16_plan(type, K, nrows, ncols, false).use ? HIP_QMM_KERNEL_F16
+                                                                           : mmq_kernel_of(type, K, nrows, ncols);
+    }
+    if (op == HIP_QMM_OP_MUL_MAT_GLU) {
+        if (ncols == 1 && K <= 32768) return HIP_QMM_KERNEL_GEMV;
+        if (glu_fuses_mmq(type, K, nrows, ncols))
+            return mmq_f16_plan(type, K, nrows, ncols, true).use ? HIP_QMM_KERNEL_F16 : HIP_QMM_KERNEL_TILE;
+        return glu_few(type, K, nrows, ncols) ? HIP_QMM_KERNEL_FEW : HIP_QMM_KERNEL_UNFUSED;
+    }
+    return -1;
+}
+
 extern "C" int hip_qmm_mul_mat(int type, const void *w, int64_t K, int64_t nrows, int64_t row_stride,
                                const float *x, int64_t ncols, int64_t x_col_stride, float *dst,
                                int64_t dst_col_stride, void *workspace, size_t workspace_size, void *stream) {

@@ -910,6 +910,11 @@ static bool few_wide(int type, int64_t K, int64_t nrows, int64_t ncols) {
            nrows * K <= ((int64_t)16 << 20) && mmq_few_whole_k(type, K, nrows, ncols);
 }
 
+int mmq_kernel_of(int type, int64_t K, int64_t nrows, int64_t ncols) {
+    if (!few_cols_type(type, K, nrows, ncols) && !few_wide(type, K, nrows, ncols)) return HIP_QMM_KERNEL_TILE;
+    return mmq_few_whole_k(type, K, nrows, ncols) ? HIP_QMM_KERNEL_FEW_WHOLE_K : HIP_QMM_KERNEL_FEW;
+}
+
 // For api.hip's f16 route: the weight checks of this dispatch, and the sum of K-split partials.
 int mmq_check_weights(int type, const void *w, int64_t K, int64_t row_stride) {
     return check_weights(type, w, K, row_stride);
@@ -941,10 +946,11 @@ extern "C" int hip_qmm_mmq(int type, const void *w, int64_t K, int64_t nrows, in
     const int bn = mmq_bn(type, K, nrows, ncols);
     const int64_t gy = (ncols + bn - 1) / bn;
     const bool few_rows = mmq_few_takes(type, K, w, row_stride) && (uintptr_t)y_qs % 16 == 0 && (uintptr_t)y_ds % 16 == 0;
-    const bool few = few_rows && (few_cols_type(type, K, nrows, ncols) || few_wide(type, K, nrows, ncols));
-    const bool whole_k = few && mmq_few_whole_k(type, K, nrows, ncols);
+    const int kernel = few_rows ? mmq_kernel_of(type, K, nrows, ncols) : HIP_QMM_KERNEL_TILE;
+    const bool few = kernel != HIP_QMM_KERNEL_TILE;
     // split K only when the caller's workspace holds the partials
-    int split = !few ? split_std(type, K, nrows, ncols) : whole_k ? 1 : mmq_few_split_k(K, nrows);
+    int split = !few ? split_std(type, K, nrows, ncols)
+                     : kernel == HIP_QMM_KERNEL_FEW_WHOLE_K ? 1 : mmq_few_split_k(K, nrows);
     if (split > 1 && (!workspace || workspace_size < (size_t)split * (size_t)nrows * (size_t)ncols * sizeof(float) ||
                       (uintptr_t)workspace % 16))
         split = 1;

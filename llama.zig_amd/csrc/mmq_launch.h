@@ -15,8 +15,10 @@ int qmm_quantize_planar(const float *x, int64_t K, int64_t ncols, int64_t x_col_
                         uint32_t keep, hipStream_t s);
 
 // mmq.hip: whether the few-column kernel takes this shape (given aligned operands),
-// the weight checks of its dispatch, and the sum of K-split partials
+// the kernel of hip_qmm_mmq on aligned operands (a HIP_QMM_KERNEL_ value, K % 256 ==
+// 0), the weight checks of its dispatch, and the sum of K-split partials
 bool few_cols_type(int type, int64_t K, int64_t nrows, int64_t ncols);
+int mmq_kernel_of(int type, int64_t K, int64_t nrows, int64_t ncols);
 int mmq_check_weights(int type, const void *w, int64_t K, int64_t row_stride);
 int mmq_add_partials(const float *partial, int split, int64_t nrows, int64_t ncols, float *dst, int64_t dst_col_stride,
                      hipStream_t s);

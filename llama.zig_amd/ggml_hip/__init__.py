@@ -48,6 +48,8 @@ def lib():
         for name in ("hip_qmm_mul_mat_workspace_preferred", "hip_qmm_mul_mat_glu_workspace_preferred"):
             getattr(L, name).restype = ctypes.c_size_t
             getattr(L, name).argtypes = [i32, i64, i64, i64]
+        L.hip_qmm_kernel.restype = i32
+        L.hip_qmm_kernel.argtypes = [i32, i32, i64, i64, i64]
         L.hip_qmm_mul_mat_uses_mmq.argtypes = [i32, i64, i64, i64]
         L.hip_qmm_mul_mat_per_column.argtypes = [i32, i64, i64, i64]
         L.hip_qmm_mul_mat_vec.restype = i32
@@ -452,6 +454,18 @@ def block_dots(qtype, w: torch.Tensor, K: int, qs: torch.Tensor):
 def workspace_size(qtype, K: int, ncols: int, nrows: int = 0) -> int:
     t = TYPE_IDS[qtype] if isinstance(qtype, str) else int(qtype)
     return int(lib().hip_qmm_mul_mat_workspace_size(t, K, nrows, ncols))
+
+
+KERNELS = ("gemv", "few", "few whole K", "tile", "f16", "unfused")
+_KERNEL_OPS = {"mul_mat": 0, "mul_mat_glu": 1, "mmq": 2}
+
+
+def kernel(op: str, qtype, K: int, nrows: int, ncols: int):
+    """The kernel (of KERNELS) that "mul_mat", "mul_mat_glu" or "mmq" runs for a shape on
+    aligned operands, None where the op does not take it; for measurement and tests."""
+    t = TYPE_IDS[qtype] if isinstance(qtype, str) else int(qtype)
+    k = int(lib().hip_qmm_kernel(_KERNEL_OPS[op], t, K, nrows, ncols))
+    return KERNELS[k] if k >= 0 else None
 
 
 def mul_mat(qtype, w: torch.Tensor, x: torch.Tensor, out=None, workspace=None):

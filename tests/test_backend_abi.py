@@ -333,3 +333,37 @@ def test_mul_mat_route_query(L):
     assert pc(q4_0, 4096, 1024, 4) == 1 and pc(q4_0, 4096, 1024, 6) == 0 and pc(q4_0, 2048, 1024, 8) == 1
     assert pc(q8_0, 2048, 1024, 8) == 1 and pc(q4_0, 2048, 1025, 2) == 0
     assert pc(q4k, 4096, 0, 2) == 0 and pc(q4k, 0, 1024, 2) == 0
+
+
+def test_kernel_query(L):
+    """hip_qmm_kernel names the kernel of each op without a device, and agrees with the
+    other queries."""
+    import ggml_hip as G
+    k = G.kernel
+    assert k("mul_mat", "Q4_K", 4096, 14336, 1) == k("mul_mat", "Q4_K", 4096, 1024, 8) == "gemv"
+    assert k("mul_mat", "Q4_K", 4096, 4096, 8) == k("mul_mat", "Q4_K", 4096, 4096, 13) == "few whole K"
+    assert k("mul_mat", "Q4_K", 4096, 14336, 8) == "few" and k("mul_mat", "Q8_0", 4100, 16, 4096) is None
+    assert k("mul_mat", "Q8_0", 4096, 14336, 100) == "tile" and k("mul_mat", "Q8_0", 4128, 4096, 100) == "gemv"
+    assert k("mul_mat", "Q4_K", 4096, 14336, 512) == "f16" and k("mul_mat", "Q4_K", 65536 + 256, 14336, 512) == "tile"
+    assert k("mul_mat_glu", "Q4_K", 4096, 14336, 1) == "gemv" and k("mul_mat_glu", "Q4_K", 4096, 14336, 4) == "few"
+    assert k("mul_mat_glu", "Q4_K", 4096, 1024, 4) == "unfused" and k("mul_mat_glu", "Q4_K", 4096, 14336, 2048) == "f16"
+    assert k("mmq", "Q4_K", 4096, 1024, 4) == "few whole K" and k("mmq", "Q4_K", 4096, 14336, 512) == "tile"
+    assert k("mmq", "Q8_0", 4096, 4096, 24) == "few whole K" and k("mmq", "Q8_0", 4128, 4096, 24) is None
+    L.hip_qmm_kernel.argtypes = [C.c_int, C.c_int] + [C.c_int64] * 3
+    assert L.hip_qmm_kernel(3, 12, 4096, 4096, 8) == L.hip_qmm_kernel(0, 1, 4096, 4096, 8) == -1
+    assert L.hip_qmm_kernel(0, 12, 4096, 0, 8) == L.hip_qmm_kernel(0, 12, 0, 4096, 8) == -1
+    for t in ("Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K", "IQ4_XS"):
+        for K in (256, 2048, 4096, 14336):
+            for rows in (1, 1024, 4096, 6144, 14336):
+                for n in (2, 4, 8, 9, 16, 17, 32, 33, 200, 2048):
+                    args = G.TYPE_IDS[t], K, rows, n
+                    if G.lib().hip_qmm_mul_mat_uses_mmq(*args):
+                        assert k("mul_mat", t, K, rows, n) != "gemv"
+                    if G.lib().hip_qmm_mul_mat_per_column(*args):
+                        assert k("mul_mat", t, K, rows, n) == "gemv"
+                    fused = k("mul_mat_glu", t, K, rows, n) != "unfused"
+                    assert fused >= bool(G.lib().hip_qmm_mul_mat_glu_fused(*args))
+                    if n > 8:
+                        assert fused == bool(G.lib().hip_qmm_mul_mat_glu_fused(*args))
+                    if k("mul_mat", t, K, rows, n) == "f16":
+                        assert G.lib().hip_qmm_mul_mat_workspace_preferred(*args) >= K // 256 * -(-n // 128) * 4 * 18432
