@@ -23,11 +23,18 @@ TYPES = {"Q4_K": O.TYPE_Q4_K, "Q5_K": O.TYPE_Q5_K, "Q6_K": O.TYPE_Q6_K, "Q8_0": 
 @pytest.mark.parametrize("nrows,K,ncols", [
     (1, 2048, 1), (15, 2048, 2), (16, 2048, 8), (17, 2048, 9),  # one workgroup and one row more; a step a wave
     (333, 4096, 7), (333, 6144, 16), (33, 6144, 17), (33, 6144, 32),  # 3 steps a wave; column tiles
+    (1537, 6144, 16), (1537, 6144, 17), (1537, 6144, 32),  # 3 steps a wave where a step has more work (Q6_K, two tiles)
     (65, 512, 5), (65, 1536, 13), (65, 2560, 31),  # fewer steps than waves; uneven parts
 ])
 def test_few_whole_k(tname, nrows, K, ncols):
     import ggml_hip as G
     t = TYPES[tname]
+    # beside it: 33 rows of 3 steps of two column tiles and 333 of Q6_K (64-row workgroups), and the
+    # tile for Q6_K above 16 columns or on rows of K % 2048 (not 16-byte aligned), for Q8_0 from 8 MiB on
+    beside = "few" if (nrows, K) == (33, 6144) or (tname, nrows, K) == ("Q6_K", 333, 6144) else "few whole K"
+    if tname == "Q6_K" and (ncols > 16 or K % 2048) or tname == "Q8_0" and nrows == 1537 and ncols > 16:
+        beside = "tile"
+    assert G.kernel("mmq", tname, K, nrows, ncols) == beside
     wq = weights_q(t, nrows, K)
     w_d = torch.from_numpy(np.array(wq)).cuda()
     x_d = torch.from_numpy(np.array(acts(ncols, K))).cuda()
@@ -61,11 +68,14 @@ def test_few_whole_k_precision(tname, ncols):
 
 
 @pytest.mark.parametrize("nrows", [12224, 12225])
+@pytest.mark.parametrize("K", [512, 1024])
 @pytest.mark.parametrize("ncols", [3, 13, 24])
-def test_few_row_limit(nrows, ncols):
-    """The last rows each form takes: 16-row workgroups up to 12224, 64-row above."""
+def test_few_row_limit(nrows, K, ncols):
+    """The last rows each form takes: 16-row workgroups up to 12224 (from 4 steps on
+    and with one column tile), 64-row above."""
     import ggml_hip as G
-    K = 512
+    whole_k = nrows == 12224 and K == 1024 and ncols <= 16
+    assert G.kernel("mmq", "Q5_K", K, nrows, ncols) == ("few whole K" if whole_k else "few")
     wq = weights_q(O.TYPE_Q5_K, nrows, K)
     w_d = torch.from_numpy(np.array(wq)).cuda()
     x_d = torch.from_numpy(np.array(acts(ncols, K))).cuda()
@@ -103,6 +113,8 @@ def test_op_route(tname, nrows, K, ncols, few):
     wq = weights_q(t, nrows, K)
     w_d = torch.from_numpy(np.array(wq)).cuda()
     x_d = torch.from_numpy(np.array(acts(ncols, K))).cuda()
+    assert G.kernel("mul_mat", tname, K, nrows, ncols) == (
+        "few whole K" if few else "gemv" if ncols <= 8 else "tile")
     got = _op(G, tname, w_d, K, x_d)
     qs, ds = G.quantize_q8_1_planar(x_d)
     gemm = G.mmq(tname, w_d, K, qs, ds).cpu().numpy()

@@ -27,11 +27,19 @@ def _lib():
 
 
 # one case per dispatch path, in decreasing workspace: MMQ with split-K
-# partials (18.8 MB), the few-column GEMM with split-K (3.3 MB), the MMQ
-# (2.4 MB), quantizer + GEMV, the one-launch 2-4 column GEMV (no scratch),
-# the one-column fused GEMV (no scratch)
-CASES = [("Q4_K", 4096, 14336, 128), ("Q4_K", 4096, 4096, 24), ("Q4_K", 4096, 4096, 512), ("Q6_K", 1024, 4096, 7),
-         ("Q8_0", 1024, 4096, 3), ("Q4_K", 4096, 4096, 1)]
+# partials (18.8 MB), the few-column GEMM without partials (3.3 MB asked, the
+# planes used), the MMQ (2.4 MB), the few-column GEMM with split-K (0.8 MB),
+# quantizer + GEMV, the one-launch 2-4 column GEMV (no scratch), the one-column
+# fused GEMV (no scratch)
+CASES = [("Q4_K", 4096, 14336, 128), ("Q4_K", 4096, 4096, 24), ("Q4_K", 4096, 4096, 512), ("Q4_K", 300, 14336, 24),
+         ("Q6_K", 1024, 4096, 7), ("Q8_0", 1024, 4096, 3), ("Q4_K", 4096, 4096, 1)]
+
+
+def test_cases_reach_their_paths():
+    G, L = _lib()
+    assert [G.kernel("mul_mat", t, K, nrows, T) for t, nrows, K, T in CASES] == [
+        "tile", "few whole K", "tile", "few", "gemv", "gemv", "gemv"]
+    assert L.hip_qmm_mmq_split_k(O.TYPE_Q4_K, 14336, 300, 24) > 1
 
 
 def test_noalloc_matches_mul_mat_on_successive_calls():
@@ -70,13 +78,13 @@ def test_noalloc_rejects_a_workspace_beyond_the_array():
 
 def test_noalloc_under_graph_capture():
     """The callers the entry point is for capture it: after one eager call
-    (which looks up the scratch array's address), two calls of different
+    (which looks up the scratch array's address), three calls of different
     shapes (the few-column GEMM with split-K partials in the scratch, then
-    the quantizer + GEMV) are captured into one HIP graph.  Every replay,
+    without, then the one-launch GEMV) are captured into one HIP graph.  Every replay,
     with eager work and synchronizations between replays, equals
     hip_qmm_mul_mat bit for bit."""
     G, L = _lib()
-    cases = [("Q4_K", 4096, 4096, 24), ("Q8_0", 1024, 4096, 3)]
+    cases = [("Q4_K", 300, 14336, 24), ("Q4_K", 4096, 4096, 24), ("Q8_0", 1024, 4096, 3)]
     ins, wants, outs = [], [], []
     for tname, nrows, K, T in cases:
         t = O.TYPE_IDS[tname]
@@ -98,7 +106,7 @@ def test_noalloc_under_graph_capture():
     g = torch.cuda.CUDAGraph()
     with torch.cuda.stream(cs):
         with torch.cuda.graph(g, stream=cs):
-            assert call(0) == 0 and call(1) == 0
+            assert all(call(i) == 0 for i in range(len(cases)))
     torch.cuda.current_stream().wait_stream(cs)
     torch.cuda.synchronize()
     for rep in range(3):
