@@ -460,19 +460,21 @@ def run_suite(name, torch, G, dev, reps, cpu=True):
                 gemv_fn = lambda i: G.mul_mat_vec(qtype, ws[i % len(ws)], Kx, qs, ds, out=out)  # noqa: E731
                 mmq_fn = lambda i: G.mmq(qtype, ws[i % len(ws)], Kx, qs, ds, out=out, workspace=mmq_ws)  # noqa: E731
                 # the op on f32 activations (hip_qmm_mul_mat: quantizer + kernel,
-                # or for one column the GEMV that quantizes in its prologue)
-                wsp = torch.empty(int(G.lib().hip_qmm_mul_mat_workspace_size(G.TYPE_IDS[qtype], Kx, M, T)),
+                # or for one column the GEMV that quantizes in its prologue), with
+                # the workspace that its wrapper and the plugin give it
+                wsp = torch.empty(int(G.lib().hip_qmm_mul_mat_workspace_preferred(G.TYPE_IDS[qtype], Kx, M, T)),
                                   dtype=torch.uint8, device=dev)
+                op_kernel = G.kernel("mul_mat", qtype, Kx, M, T)
                 op_fn = lambda i: G.mul_mat(qtype, ws[i % len(ws)], x, out=out, workspace=wsp)  # noqa: E731
                 if 2 <= T <= 8 and G.lib().hip_qmm_mul_mat_per_column(G.TYPE_IDS[qtype], Kx, M, T):
                     # one launch: the one-column kernel per column, quantizing in the kernel
                     fn, kern = op_fn, "gemv one-column kernel per column"
-                elif T <= 8 and not G.lib().hip_qmm_mul_mat_uses_mmq(G.TYPE_IDS[qtype], Kx, M, T):
+                elif T <= 8 and op_kernel == "gemv":
                     fn, kern = gemv_fn, "gemv"
                 else:
                     fn, kern = mmq_fn, ("mmq few-column" if T <= 8 else "mmq")
                 ms = event_time_batch(torch, fn, n)
-                extra = {}
+                extra = {"op_kernel": op_kernel}  # "f16" where the op runs that GEMM instead of the MMQ timed here
                 if T <= 8 and kern != "gemv":
                     extra["gemv_us"] = round(event_time_batch(torch, gemv_fn, n) * 1e3, 3)
                 if name == "few":
@@ -661,9 +663,10 @@ def run_suite(name, torch, G, dev, reps, cpu=True):
             u = torch.empty_like(out)
             g = torch.empty_like(out)
             t = G.TYPE_IDS["Q4_K"]
-            wsf = torch.empty(max(1, int(G.lib().hip_qmm_mul_mat_glu_workspace_size(t, Kx, M, T))),
+            wsf = torch.empty(max(1, int(G.lib().hip_qmm_mul_mat_glu_workspace_preferred(t, Kx, M, T))),
                               dtype=torch.uint8, device=dev)
-            wsu = torch.empty(int(G.lib().hip_qmm_mul_mat_workspace_size(t, Kx, M, T)), dtype=torch.uint8, device=dev)
+            wsu = torch.empty(int(G.lib().hip_qmm_mul_mat_workspace_preferred(t, Kx, M, T)), dtype=torch.uint8,
+                              device=dev)
 
             def fused(i):
                 G.mul_mat_glu("Q4_K", wu[i % n], wg[i % n], x, "SWIGLU", out=out, workspace=wsf)
@@ -677,6 +680,7 @@ def run_suite(name, torch, G, dev, reps, cpu=True):
             msu = event_time_batch(torch, unfused, n * reps)
             ops = 2.0 * 2 * M * Kx * T
             emit({"suite": name, "kernel": "gate+up+swiglu fused MMQ", "type": "Q4_K", "shape": f"2x{M}x{Kx}",
+                  "op_kernel": G.kernel("mul_mat_glu", "Q4_K", Kx, M, T),
                   "label": "llama3-8b ffn_gate/up", "T": T, "fused": bool(G.lib().hip_qmm_mul_mat_glu_fused(
                       t, Kx, M, T)), "us": round(msf * 1e3, 3), "unfused_us": round(msu * 1e3, 3),
                   "TOPS": round(ops / msf / 1e9, 2), "int8_frac": round(ops / msf / 1e9 / INT8_PEAK_TOPS, 4)})
@@ -925,7 +929,8 @@ def main():
         mmq = lambda i: G.mmq("Q4_K", weights[i % ncopy], K, qst, dst_, out=outt)  # noqa: E731
         mmq_avg_ms, mmq_reps = event_time_replays(torch, mmq, n_m)
         _, mmq_med_ms = event_time_kernel(torch, mmq, n_m)
-        wst = torch.empty(G.workspace_size("Q4_K", K, T_MMQ, M), dtype=torch.uint8, device=dev)
+        wst = torch.empty(int(G.lib().hip_qmm_mul_mat_workspace_preferred(G.TYPE_IDS["Q4_K"], K, M, T_MMQ)),
+                          dtype=torch.uint8, device=dev)
         op = lambda i: G.mul_mat("Q4_K", weights[i % ncopy], xt, out=outt, workspace=wst)  # noqa: E731
         op_avg_ms, op_reps = event_time_replays(torch, op, n_m)
         gpu_mmq_out = G.mul_mat("Q4_K", weights[0], xt).cpu().numpy()
@@ -938,7 +943,8 @@ def main():
             "replays_us": [round(v * 1e3, 2) for v in mmq_reps],
             "op_avg_us": round(op_avg_ms * 1e3, 2),
             "op_replays_us": [round(v * 1e3, 2) for v in op_reps],
-            "op": "mul_mat on f32 columns: Q8_1 quantizer + the MMQ",
+            "op": "mul_mat on f32 columns with the workspace its wrapper gives it: quantizer + the "
+                  f"{G.kernel('mul_mat', 'Q4_K', K, M, T_MMQ)} GEMM",
             "roofline": {"bound": "mfma", "achieved": round(tops, 2), "peak": INT8_PEAK_TOPS, "unit": "TOP/s",
                          "frac": round(tops / INT8_PEAK_TOPS, 4), "traffic": None,
                          "algorithmic_ops": ops, "algorithmic_bytes_read": w_bytes + T_MMQ * (G.padded_k(K) * 9 // 8),
