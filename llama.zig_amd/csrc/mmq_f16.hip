@@ -1,5 +1,5 @@
-// mmq_f16.hip -- prefill GEMM of the Q4_K and Q5_K weights on the f16 matrix
-// cores, exact in its integer block products.
+// mmq_f16.hip -- prefill GEMM of the Q4_K, Q5_K and Q6_K weights on the f16
+// matrix cores, exact in its integer block products.
 //
 // The int8 MMQ (mmq_q4k_dma.hip, mmq_q5k_dma.hip) is bound by vector work: per
 // output and 32-deep block it converts an int32 dot (v_cvt_f32_i32 takes 4.2
@@ -12,14 +12,15 @@
 // 32-deep block exactly in f32 (|sc * dot| < 2^24), and an output costs one FMA
 // with the column's d8 (kept as d8 * 2^24).  d and the min term are applied
 // once per super-block as in the int8 kernels, in the same order, so the
-// outputs equal the unsplit int8 MMQ's bit for bit.
+// outputs of Q4_K and Q5_K equal the unsplit int8 MMQ's bit for bit (Q6_K's
+// scales take two operands each, see Raw<TYPE_Q6_K>).
 //
 // Per 32x32 tile and 32-deep block (one wave, two waves per SIMD) the matrix
 // cores take 67 cycles, the FMAs 43, the super-block terms 21, decoding 18 (at
-// four column tiles a wave), LDS reads 14 and transfers 11: measured with each
-// part removed, they add up (162 cycles; the int8 kernel about 220).  What is
-// left is the sum of matrix and vector work and the clock, which falls to
-// 1.95-2.1 GHz under it.
+// four column tiles a wave), LDS reads 14 and transfers 11, each measured as
+// what its removal saves: 174 cycles in sum where the whole takes 162, so they
+// hardly overlap (the int8 kernel takes about 220).  What is left is the sum of
+// matrix and vector work and the clock, which falls to 1.95-2.1 GHz under it.
 //
 // Layout.  A workgroup of NW waves takes 32 * NW weight rows by 32 * NCT
 // columns; every wave holds 32 rows: its super-block is decoded once into 16
