@@ -350,7 +350,8 @@ __global__ __launch_bounds__((KH * FewGeo<TYPE, NW, NCT, PACK>::NT), (few_waves<
     // MFMA's in lanes 0-31; the other slots add nothing because one side is zero and
     // the other finite.  The columns' s8 must not stand beside a zero: a block whose
     // 32 activations sum past 65504 (each 3000) has an infinite s8 with a finite d8,
-    // and zero times it is NaN.  So the scale MFMA's B holds d8 only; Q4_K and Q5_K
+    // and zero times it is NaN.  So the scale MFMA's B holds d8 only (infinite itself
+    // only where an activation is past 8.3 million: 127 * 65504); Q4_K and Q5_K
     // above 8 columns keep the headers as stored, since their min term is infinite
     // with such an s8 anyway (masked they took 2-4 % longer, Q5_K's whole-K form, whose
     // registers then spill, 8-17 %).
