@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the MI355X quantized-matmul path (one GPU).
 
-Metric (BASELINE.json): "Q4_K GEMV GB/s (% HBM peak) @14336x4096 b=1; MMQ
+Metric: "Q4_K GEMV GB/s (% HBM peak) @14336x4096 b=1; MMQ
 int8 TOPS @b=512".  A step is one ggml_mul_mat of the headline decode shape:
 the Q4_K weight 14336x4096 times one f32 activation column; for one column
 the op runs a single kernel, the GEMV with the Q8_1 quantization fused in.
@@ -188,7 +188,7 @@ def host_info(threads):
     except (AttributeError, OSError):
         allowed = None
     return {"cpu_model": model, "host_logical_cpus": os.cpu_count(), "cpus_allowed": allowed, "threads": threads,
-            "thread_cap": "16: the GPU box's CPU share for one GPU"}
+            "thread_cap": "16: the CPU share of one GPU"}
 
 
 def reference_inputs(T):
@@ -404,7 +404,7 @@ def cpu_suite_case(qtype, w_dev, M, Kx, x_dev):
 
 
 def run_suite(name, torch, G, dev, reps, cpu=True):
-    """Kernel-level measurements over the configs of BASELINE.json, one JSON
+    """Kernel-level measurements over the benchmark's configurations, one JSON
     line per case (device time from a HIP graph of launches between events,
     weights rotated over > 2 x the Infinity Cache), with the reference CPU
     path's time for the same case beside it (cpu_us, see cpu_suite_case)."""
@@ -482,7 +482,9 @@ def run_suite(name, torch, G, dev, reps, cpu=True):
                     # to 8 columns)
                     few_fn = lambda i: G.mmq(qtype, ws[i % len(ws)], Kx, qs, ds, out=out, workspace=mmq_ws)  # noqa: E731
                     extra["few_us"] = round(event_time_batch(torch, few_fn, n) * 1e3, 3)
-                    extra["few_split"] = int(G.lib().hip_qmm_mmq_split_k(G.TYPE_IDS[qtype], Kx, M, T))
+                    extra["few_kernel"] = G.kernel("mmq", qtype, Kx, M, T)
+                    extra["few_split"] = (1 if extra["few_kernel"] == "few whole K" else
+                                          int(G.lib().hip_qmm_mmq_split_k(G.TYPE_IDS[qtype], Kx, M, T)))
                     if qtype not in ("Q4_K", "Q5_K") and T > 8:
                         if T == 9:
                             off = []
